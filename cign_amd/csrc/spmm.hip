@@ -7,8 +7,17 @@
 //
 // Layout: x, add, y are row-major [n_rows, ld] (fp32 or bf16 storage, fp32
 // accumulation); P is CSR with int32 row pointer / column index and fp32
-// values. One launch handles a column tile of at most 256 16-byte chunks per
-// row; wider matrices are tiled by the host.
+// values. One launch handles at most 256 16-byte chunks per row; wider
+// matrices take several launches.
+//
+// A gather is bound by the cache lines it can have in flight, so by their
+// latency: a launch of wide rows is split into column tiles that stay on
+// their XCDs (workgroup ids go round-robin to the 8 XCDs), so that an XCD's
+// 4 MB L2 holds more of the rows' slices it gathers (launch_all). 24,492
+// nodes, 220,420 entries, fp32, us per hop forward / backward, untiled ->
+// tiled: D = 512 56.1 / 61.9 -> 48.0 / 54.5 (8 tiles of 256 bytes), 384 40.5 /
+// 44.0 -> 36.5 / 39.8, 256 26.6 / 28.7 -> 24.6 / 26.6, 192 21.2 / 22.6 ->
+// 19.4 / 20.9; 2,000 nodes, D = 512: 14.4 -> 8.5 (too few wavefronts untiled).
 //
 // A row's output is owned by a group of L lanes (L = power of two covering
 // the tile's chunks, 16-byte loads, lane l owns chunks l, l + L, ...). Three
@@ -31,6 +40,58 @@
 #include "schedule.h"
 
 namespace cign {
+
+// Values of rows that are not 16-byte aligned (odd widths, views): the same
+// 16-byte accesses with the alignment of one value. Against one value a lane
+// (24,492 nodes): fp32 D = 33 12.8 -> 7.9 us, 115 17.8 -> 13.7, 333 51.1 ->
+// 37.5; bf16 D = 333 120 -> 29, 334 120 -> 25.
+struct f32u {
+  float v;
+};
+struct bf16u {
+  uint16_t bits;
+};
+__device__ __forceinline__ float to_f32(f32u v) { return v.v; }
+__device__ __forceinline__ float to_f32(bf16u v) { return __uint_as_float(static_cast<uint32_t>(v.bits) << 16); }
+template <>
+__device__ __forceinline__ f32u from_f32<f32u>(float f) { return f32u{f}; }
+template <>
+__device__ __forceinline__ bf16u from_f32<bf16u>(float f) { return bf16u{from_f32<bf16>(f).bits}; }
+
+template <>
+struct Chunk<f32u, 4> {
+  using Raw = float4;
+  typedef float Vec __attribute__((ext_vector_type(4), aligned(4)));
+  static __device__ __forceinline__ Raw load_raw(const f32u* p) {
+    const Vec q = *reinterpret_cast<const Vec*>(p);
+    return make_float4(q.x, q.y, q.z, q.w);
+  }
+  static __device__ __forceinline__ Raw zero_raw() { return make_float4(0.0f, 0.0f, 0.0f, 0.0f); }
+  static __device__ __forceinline__ void unpack(const Raw& q, float (&v)[4]) { Chunk<float, 4>::unpack(q, v); }
+  static __device__ __forceinline__ void store(f32u* p, const float (&v)[4]) {
+    *reinterpret_cast<Vec*>(p) = Vec{v[0], v[1], v[2], v[3]};
+  }
+};
+
+template <>
+struct Chunk<bf16u, 8> {
+  using Raw = uint4;
+  typedef uint32_t Vec __attribute__((ext_vector_type(4), aligned(2)));
+  static __device__ __forceinline__ Raw load_raw(const bf16u* p) {
+    const Vec q = *reinterpret_cast<const Vec*>(p);
+    return make_uint4(q.x, q.y, q.z, q.w);
+  }
+  static __device__ __forceinline__ Raw zero_raw() { return make_uint4(0u, 0u, 0u, 0u); }
+  static __device__ __forceinline__ void unpack(const Raw& q, float (&v)[8]) { Chunk<bf16, 8>::unpack(q, v); }
+  static __device__ __forceinline__ void store(bf16u* p, const float (&v)[8]) {
+    uint32_t w[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      w[i] = from_f32<bf16>(v[2 * i]).bits | (static_cast<uint32_t>(from_f32<bf16>(v[2 * i + 1]).bits) << 16);
+    *reinterpret_cast<Vec*>(p) = Vec{w[0], w[1], w[2], w[3]};
+  }
+};
+
 namespace {
 
 // Workgroup shape of the SpMM: kSpmmWaves wavefronts; a heavy-row segment is
@@ -53,11 +114,15 @@ constexpr int kSpmmBlock = kSpmmWaves * kWave;
 constexpr int kTile = 64;
 constexpr int kSegEdges = kSpmmWaves * kTile;
 
-template <typename T, int W, int VPL>
+template <typename T, int W, int VPL, bool TILED>
 struct SpmmArgs {
   int ld;       // row stride of x / add / y (elements)
-  int c0;       // first column of this tile
-  int nch;      // chunks (of W elements) in this tile
+  int c0;       // first column of the launch; in the kernel, of the workgroup's tile
+  int nch;      // chunks (of W elements) of the launch; in the kernel, of the tile
+  int tch;      // chunks per tile
+  int lgT;      // log2 of the tile slots workgroup ids are dealt over
+  int n_tile;   // tiles (slots past them exit)
+  int width;    // columns of the launch (row stride of `partial`)
   int L;        // lanes per group (power of two, L * VPL >= nch)
   int lgL;      // log2(L)
   int n_mid;    // light rows processed one per wavefront (the first n_mid)
@@ -67,11 +132,11 @@ struct SpmmArgs {
   const T* x;
   const T* add;  // may be null
   T* y;
-  float* partial;     // [n_seg, nch * W] scratch for multi-segment rows
+  float* partial;     // [n_seg, width] scratch for multi-segment rows
   int32_t* counters;  // [n_hrow], zero on entry, left zero on exit
 };
 
-template <typename T, int W, int VPL>
+template <int VPL, int W>
 __device__ __forceinline__ void zero(float (&acc)[VPL][W]) {
 #pragma unroll
   for (int v = 0; v < VPL; ++v)
@@ -79,15 +144,25 @@ __device__ __forceinline__ void zero(float (&acc)[VPL][W]) {
     for (int w = 0; w < W; ++w) acc[v][w] = 0.0f;
 }
 
+// First column of the tile's chunk c within its row, from a.c0. Where the row
+// is no whole number of chunks, the last chunk of the row ends at the row's
+// end and repeats columns of the one before it (the same sums, in the same
+// order, stored twice).
+template <typename T, int W, int VPL, bool TILED>
+__device__ __forceinline__ int chunk_col(const SpmmArgs<T, W, VPL, TILED>& a, int c) {
+  if constexpr (std::is_same<T, f32u>::value || std::is_same<T, bf16u>::value) return min(c * W, a.ld - W - a.c0);
+  return c * W;
+}
+
 // Raw chunks of x[j] owned by lane gl (zero past the tile).
-template <typename T, int W, int VPL>
-__device__ __forceinline__ void load_row(const SpmmArgs<T, W, VPL>& a, int j, int gl,
+template <typename T, int W, int VPL, bool TILED>
+__device__ __forceinline__ void load_row(const SpmmArgs<T, W, VPL, TILED>& a, int j, int gl,
                                          typename Chunk<T, W>::Raw (&buf)[VPL]) {
   const T* base = a.x + static_cast<int64_t>(j) * a.ld + a.c0;
 #pragma unroll
   for (int v = 0; v < VPL; ++v) {
     const int c = gl + (v << a.lgL);
-    buf[v] = c < a.nch ? Chunk<T, W>::load_raw(base + c * W) : Chunk<T, W>::zero_raw();
+    buf[v] = c < a.nch ? Chunk<T, W>::load_raw(base + chunk_col(a, c)) : Chunk<T, W>::zero_raw();
   }
 }
 
@@ -95,9 +170,9 @@ __device__ __forceinline__ void load_row(const SpmmArgs<T, W, VPL>& a, int j, in
 // valid while u < cnt, whose column index and weight lane (base + u) holds in
 // jj / vv. Every gather of a batch is issued before any is consumed; slots
 // past the end reload an edge of the group with weight 0.
-template <typename T, int W, int VPL>
+template <typename T, int W, int VPL, bool TILED>
 struct SpmmBatches {
-  const SpmmArgs<T, W, VPL>& a;
+  const SpmmArgs<T, W, VPL, TILED>& a;
   int jj;
   float vv;
   int base, first, step, cnt, gl;
@@ -135,10 +210,10 @@ __device__ __forceinline__ int wave_max_over_groups(int v, int L) {
 
 // Gathers `need` (wave-uniform) slots per lane group, at most kSpmmInflight
 // chunks in flight per lane.
-template <typename T, int W, int VPL>
-__device__ __forceinline__ void gather(const SpmmArgs<T, W, VPL>& a, int jj, float vv, int base, int first, int step,
+template <typename T, int W, int VPL, bool TILED>
+__device__ __forceinline__ void gather(const SpmmArgs<T, W, VPL, TILED>& a, int jj, float vv, int base, int first, int step,
                                        int cnt, int need, int gl, float (&acc)[VPL][W]) {
-  SpmmBatches<T, W, VPL> sb{a, jj, vv, base, first, step, cnt, gl, acc};
+  SpmmBatches<T, W, VPL, TILED> sb{a, jj, vv, base, first, step, cnt, gl, acc};
   for_batches<(kSpmmInflight / VPL > 0 ? kSpmmInflight / VPL : 1)>(need, sb);
 }
 
@@ -146,28 +221,28 @@ __device__ __forceinline__ void gather(const SpmmArgs<T, W, VPL>& a, int jj, flo
 // before its gathers (at the write they were one more memory round trip
 // after the gathers, on every hop with a fused add). Chunks past the tile
 // read the tile's last chunk (never used).
-template <typename T, int W, int VPL>
+template <typename T, int W, int VPL, bool TILED>
 struct AddRow {
   typename Chunk<T, W>::Raw raw[VPL];
-  __device__ __forceinline__ void load(const SpmmArgs<T, W, VPL>& a, int row, int gl) {
+  __device__ __forceinline__ void load(const SpmmArgs<T, W, VPL, TILED>& a, int row, int gl) {
     if (!a.add) return;  // uniform
     const T* base = a.add + static_cast<int64_t>(row) * a.ld + a.c0;
 #pragma unroll
     for (int v = 0; v < VPL; ++v) {
       const int c = min(gl + (v << a.lgL), a.nch - 1);
-      raw[v] = Chunk<T, W>::load_raw(base + c * W);
+  raw[v] = Chunk<T, W>::load_raw(base + chunk_col(a, c));
     }
   }
 };
 
-template <typename T, int W, int VPL>
-__device__ __forceinline__ void write_row(const SpmmArgs<T, W, VPL>& a, int row, int gl, const float (&acc)[VPL][W],
-                                          const AddRow<T, W, VPL>& ar) {
+template <typename T, int W, int VPL, bool TILED>
+__device__ __forceinline__ void write_row(const SpmmArgs<T, W, VPL, TILED>& a, int row, int gl, const float (&acc)[VPL][W],
+                                          const AddRow<T, W, VPL, TILED>& ar) {
 #pragma unroll
   for (int v = 0; v < VPL; ++v) {
     const int c = gl + (v << a.lgL);
     if (c < a.nch) {
-      const int64_t off = static_cast<int64_t>(row) * a.ld + a.c0 + c * W;
+      const int64_t off = static_cast<int64_t>(row) * a.ld + a.c0 + chunk_col(a, c);
       float out[W];
 #pragma unroll
       for (int w = 0; w < W; ++w) out[w] = acc[v][w];
@@ -182,16 +257,26 @@ __device__ __forceinline__ void write_row(const SpmmArgs<T, W, VPL>& a, int row,
   }
 }
 
-template <typename T, int W, int VPL>
-__global__ __launch_bounds__(kSpmmBlock) void spmm_kernel(SpmmArgs<T, W, VPL> a, Sched s) {
+template <typename T, int W, int VPL, bool TILED>
+__global__ __launch_bounds__(kSpmmBlock) void spmm_kernel(SpmmArgs<T, W, VPL, TILED> a, Sched s) {
   const int lane = lane_id();
   const int wave = wave_id();
   const int gl = lane & (a.L - 1);
   const int G = kWave >> a.lgL;
   const int g = lane >> a.lgL;
+  // Workgroup ids go round-robin to the XCDs, so a tile stays on the same
+  // XCDs (launch_all).
   int b = blockIdx.x;
+  const int launch_c0 = a.c0;
+  if constexpr (TILED) {
+    const int tile = b & ((1 << a.lgT) - 1);
+    b >>= a.lgT;
+    if (tile >= a.n_tile) return;
+    a.c0 += tile * a.tch * W;
+    a.nch = min(a.tch, a.nch - tile * a.tch);
+  }
   float acc[VPL][W];
-  zero<T, W, VPL>(acc);
+  zero(acc);
 
   if (b >= s.n_seg) {
     b -= s.n_seg;
@@ -205,7 +290,7 @@ __global__ __launch_bounds__(kSpmmBlock) void spmm_kernel(SpmmArgs<T, W, VPL> a,
       const bool mine = lane < deg;
       const int jj = mine ? a.col[r.y + lane] : 0;
       const float vv = mine ? a.val[r.y + lane] : 0.0f;
-      AddRow<T, W, VPL> ar;
+      AddRow<T, W, VPL, TILED> ar;
       ar.load(a, r.x, gl);
       gather(a, jj, vv, 0, g, G, deg, (deg + G - 1) / G, gl, acc);
       sum_across_n(acc, a.L);
@@ -220,9 +305,12 @@ __global__ __launch_bounds__(kSpmmBlock) void spmm_kernel(SpmmArgs<T, W, VPL> a,
     const bool mine = gl < deg;
     const int jj = mine ? a.col[r.y + gl] : 0;
     const float vv = mine ? a.val[r.y + gl] : 0.0f;
-    AddRow<T, W, VPL> ar;
+    AddRow<T, W, VPL, TILED> ar;
     ar.load(a, r.x, gl);  // (row 0 for a group with no row: read, unused)
     gather(a, jj, vv, g << a.lgL, 0, 1, deg, wave_max_over_groups(deg, a.L), gl, acc);
+    // A group's slots past its row's end reload an edge of that row; a row with
+    // no edge has read another row's.
+    if (deg == 0) zero(acc);
     if (has) write_row(a, r.x, gl, acc, ar);
     return;
   }
@@ -249,7 +337,11 @@ __global__ __launch_bounds__(kSpmmBlock) void spmm_kernel(SpmmArgs<T, W, VPL> a,
     vv = vn;
   }
   sum_across_n(acc, a.L);
-  const int width = a.nch * W;
+  // Columns of the tile; column c is value red_at(c) of its chunks.
+  const int width = min(a.nch * W, a.ld - a.c0);
+  const int full = (a.nch - 1) * W;
+  const int skip = a.nch * W - width;
+  const auto red_at = [&](int c) { return c < full ? c : c + skip; };
   if (lane < a.L) {
 #pragma unroll
     for (int v = 0; v < VPL; ++v) {
@@ -265,25 +357,27 @@ __global__ __launch_bounds__(kSpmmBlock) void spmm_kernel(SpmmArgs<T, W, VPL> a,
     for (int c = threadIdx.x; c < width; c += kSpmmBlock) {
       float t = 0.0f;
 #pragma unroll
-      for (int v = 0; v < kSpmmWaves; ++v) t += red[v][c];
+      for (int v = 0; v < kSpmmWaves; ++v) t += red[v][red_at(c)];
       const int64_t off = static_cast<int64_t>(row) * a.ld + a.c0 + c;
       if (a.add) t += to_f32(a.add[off]);
       a.y[off] = from_f32<T>(t);
     }
     return;
   }
-  float* part = a.partial + static_cast<int64_t>(b) * width;
+  // The last of the row's workgroups, over all of its tiles, adds the
+  // partials of the whole row (one counter per row).
+  float* part = a.partial + static_cast<int64_t>(b) * a.width + (a.c0 - launch_c0);
   for (int c = threadIdx.x; c < width; c += kSpmmBlock) {
     float t = 0.0f;
 #pragma unroll
-    for (int v = 0; v < kSpmmWaves; ++v) t += red[v][c];
+    for (int v = 0; v < kSpmmWaves; ++v) t += red[v][red_at(c)];
     st_agent(part + c, t);
   }
-  if (!arrive_last(a.counters + sg.w, hr.y, &flag)) return;
-  for (int c = threadIdx.x; c < width; c += kSpmmBlock) {
+  if (!arrive_last(a.counters + sg.w, hr.y * a.n_tile, &flag)) return;
+  for (int c = threadIdx.x; c < a.width; c += kSpmmBlock) {
     float t = 0.0f;
-    for (int q = 0; q < hr.y; ++q) t += ld_agent(a.partial + static_cast<int64_t>(hr.x + q) * width + c);
-    const int64_t off = static_cast<int64_t>(row) * a.ld + a.c0 + c;
+    for (int q = 0; q < hr.y; ++q) t += ld_agent(a.partial + static_cast<int64_t>(hr.x + q) * a.width + c);
+    const int64_t off = static_cast<int64_t>(row) * a.ld + launch_c0 + c;
     if (a.add) t += to_f32(a.add[off]);
     a.y[off] = from_f32<T>(t);
   }
@@ -302,15 +396,19 @@ struct SchedInfo {
 
 inline SchedInfo read_info(const int32_t* hdr) { return SchedInfo{hdr, hdr[0], hdr[1], hdr[2]}; }
 
-template <typename T, int W, int VPL>
-int launch_tile(hipStream_t stream, const Sched& s, const SchedInfo& info, int ld, int c0, int nch,
-                const int32_t* col, const float* val, const T* x, const T* add, T* y, float* partial,
-                int32_t* counters) {
-  SpmmArgs<T, W, VPL> a;
+template <typename T, int W, int VPL, bool TILED>
+int launch_tiles(hipStream_t stream, const Sched& s, const SchedInfo& info, int ld, int c0, int nch, int tch, int lgT,
+                 const int32_t* col, const float* val, const T* x, const T* add, T* y, float* partial,
+                 int32_t* counters) {
+  SpmmArgs<T, W, VPL, TILED> a;
   a.ld = ld;
   a.c0 = c0;
   a.nch = nch;
-  const int lanes_needed = (nch + VPL - 1) / VPL;
+  a.tch = tch;
+  a.lgT = lgT;
+  a.n_tile = (nch + tch - 1) / tch;
+  a.width = min(nch * W, ld - c0);
+  const int lanes_needed = (tch + VPL - 1) / VPL;
   a.lgL = ilog2(lanes_needed < 1 ? 1 : lanes_needed);
   a.L = 1 << a.lgL;
   a.col = col;
@@ -328,27 +426,50 @@ int launch_tile(hipStream_t stream, const Sched& s, const SchedInfo& info, int l
   a.mid_blocks = (n_mid + kSpmmWaves - 1) / kSpmmWaves;
   const int n_tiny = info.n_light - n_mid;
   const int tiny_blocks = (n_tiny + kSpmmWaves * G - 1) / (kSpmmWaves * G);
-  const int blocks = s.n_seg + a.mid_blocks + tiny_blocks;
+  const int64_t blocks = static_cast<int64_t>(s.n_seg + a.mid_blocks + tiny_blocks) << lgT;
   if (blocks == 0) return kOk;
-  hipLaunchKernelGGL((spmm_kernel<T, W, VPL>), dim3(blocks), dim3(kSpmmBlock), 0, stream, a, s);
+  if (blocks > INT32_MAX) return set_error(kInvalid, "cign_spmm: %lld workgroups", static_cast<long long>(blocks));
+  hipLaunchKernelGGL((spmm_kernel<T, W, VPL, TILED>), dim3(static_cast<unsigned>(blocks)), dim3(kSpmmBlock), 0, stream, a, s);
   return check_launch("cign_spmm");
 }
 
 template <typename T, int W>
 int launch_all(hipStream_t stream, const Sched& s, const SchedInfo& info, int ld, const int32_t* col,
                const float* val, const T* x, const T* add, T* y, float* partial, int32_t* counters) {
-  const int total_ch = ld / W;
-  constexpr int kMaxCh = kWave * 4;  // chunks per tile
+  const int total_ch = (ld + W - 1) / W;
+  constexpr int kMaxCh = kWave * 4;  // chunks per launch
+  constexpr int kChunkBytes = static_cast<int>(sizeof(T)) * W;
+  constexpr bool kTiles = W > 1 && (std::is_same<T, float>::value || std::is_same<T, bf16>::value);
+  constexpr int kTileBytes = sizeof(T) == 4 ? 256 : 512;
   for (int ch0 = 0; ch0 < total_ch; ch0 += kMaxCh) {
     const int nch = min(kMaxCh, total_ch - ch0);
-    int rc;
-    if (nch <= kWave && kSpmmMinVpl <= 1) {
-      rc = launch_tile<T, W, 1>(stream, s, info, ld, ch0 * W, nch, col, val, x, add, y, partial, counters);
-    } else if (nch <= 2 * kWave && kSpmmMinVpl <= 2) {
-      rc = launch_tile<T, W, 2>(stream, s, info, ld, ch0 * W, nch, col, val, x, add, y, partial, counters);
-    } else {
-      rc = launch_tile<T, W, 4>(stream, s, info, ld, ch0 * W, nch, col, val, x, add, y, partial, counters);
+    const int c0 = ch0 * W;
+    // Column tiles of one launch: up to 8, none narrower than kTileBytes (a
+    // bf16 lane unpacks twice the values of a load, so its narrow tiles cost
+    // more issue than they save latency: D = 512 29.4 us untiled, 27.3 in two
+    // tiles of 512 bytes, 29.2 in four). Rows of at most 512 bytes stay whole
+    // (fp32 D = 128: 13.5 us either way), and so do rows that are no whole
+    // number of 128-byte lines, whose tiles would share lines (fp32 D = 200:
+    // 22.8 us whole, 24.0 in two tiles).
+    int lgT = 0;
+    if constexpr (kTiles) {
+      if (nch * kChunkBytes > 512 && (ld * static_cast<int>(sizeof(T))) % 128 == 0)
+        while (lgT < 3 && (nch >> (lgT + 1)) * kChunkBytes >= kTileBytes) ++lgT;
     }
+    const int tch = (nch + (1 << lgT) - 1) >> lgT;
+    const int vpl = tch <= (lgT == 0 ? kWave : 16) ? 1 : tch <= 2 * kWave ? 2 : 4;
+    int rc = kOk;
+#define CIGN_SPMM_LAUNCH(VPL, TILED)                                                                             \
+  rc = launch_tiles<T, W, VPL, TILED>(stream, s, info, ld, c0, nch, tch, lgT, col, val, x, add, y, partial, counters)
+    if (lgT == 0) {
+      if (vpl == 1) CIGN_SPMM_LAUNCH(1, false);
+      else if (vpl == 2) CIGN_SPMM_LAUNCH(2, false);
+      else CIGN_SPMM_LAUNCH(4, false);
+    } else if constexpr (kTiles) {
+      if (vpl == 1) CIGN_SPMM_LAUNCH(1, true);
+      else CIGN_SPMM_LAUNCH(2, true);
+    }
+#undef CIGN_SPMM_LAUNCH
     if (rc != kOk) return rc;
   }
   return kOk;
@@ -365,6 +486,11 @@ int spmm_dispatch(hipStream_t stream, const Sched& s, const SchedInfo& info, int
                        (add == nullptr || reinterpret_cast<uintptr_t>(add) % 16 == 0);
   if (d % kVec == 0 && aligned) {
     return launch_all<T, kVec>(stream, s, info, d, col, val, xt, at, yt, partial, counters);
+  }
+  if (d >= kVec) {
+    using U = typename std::conditional<sizeof(T) == 4, f32u, bf16u>::type;
+    return launch_all<U, kVec>(stream, s, info, d, col, val, reinterpret_cast<const U*>(xt),
+                               reinterpret_cast<const U*>(at), reinterpret_cast<U*>(yt), partial, counters);
   }
   return launch_all<T, 1>(stream, s, info, d, col, val, xt, at, yt, partial, counters);
 }

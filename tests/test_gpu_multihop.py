@@ -267,3 +267,42 @@ def test_spmm_big_hubs_segment_sizes(seg_edges, dtype, d):
         xn = x.double().cpu().numpy()
         assert_within(y.double().cpu().numpy(), ref, _bf16_hop_bound(pv, xn, ref), "spmm bf16")
     assert int(parts.sched.counters.abs().sum()) == 0
+
+
+# Widths at the edges of the column tiling (rows of 512 bytes and less whole,
+# then 2, 4 and 8 tiles, more than one launch) and rows without 16-byte
+# alignment (the last chunk overlaps the one before it).
+@pytest.mark.parametrize("dtype,d", [(torch.float32, d) for d in
+                                     (4, 5, 33, 63, 128, 129, 160, 192, 333, 384, 512, 544, 1023, 1027, 2048)] +
+                         [(torch.bfloat16, d) for d in (8, 9, 63, 254, 256, 320, 334, 512, 1024, 2049)])
+def test_spmm_column_tiles_and_unaligned_rows(dtype, d):
+    from cign_amd.graph import HipCsr
+    from cign_amd.schedule import build_row_schedule
+
+    print(f"spmm tiles dtype={dtype} d={d}", flush=True)
+    rng = np.random.default_rng(d)
+    n = 700
+    deg = rng.integers(0, 30, n)
+    deg[[3, 650]] = [690, 300]  # several segments, one segment
+    deg[[0, 1, 699]] = 0
+    rp = np.concatenate([[0], np.cumsum(deg)])
+    # node 0 is no row's source and holds no number
+    col = np.concatenate([1 + np.sort(rng.choice(n - 1, size=int(k), replace=False)) for k in deg]).astype(np.int64)
+    val = (rng.random(col.size) / np.repeat(np.maximum(deg, 1), deg)).astype(np.float32)
+    crow = torch.from_numpy(rp).cuda()
+    parts = HipCsr(torch.sparse_csr_tensor(crow, torch.from_numpy(col).cuda(), torch.from_numpy(val).cuda(),
+                                           size=(n, n)))
+    parts.sched = build_row_schedule(crow, seg_edges=256)
+    x, add = _rand((n, d), dtype, 3), _rand((n, d), dtype, 4)
+    x[0] = float("nan")
+    p = (rp, col, val.astype(np.float64))
+    xn, an = x.double().cpu().numpy(), add.double().cpu().numpy()
+    xn[0] = 0.0
+    for a, add_n in ((None, None), (add, an)):
+        y = parts.spmm(x, add=a)
+        ref = O.spmm(*p, xn, add=add_n)
+        if dtype == torch.float32:
+            assert_close(y.cpu().numpy(), ref, name="spmm", **F32_TOL)
+        else:
+            assert_within(y.double().cpu().numpy(), ref, _bf16_hop_bound(p, xn, ref, add=add_n), "spmm bf16")
+    assert int(parts.sched.counters.abs().sum()) == 0
