@@ -89,34 +89,45 @@ __global__ void zero_floats(float* p, int n) {
 }
 
 // Feature-layout geometry of a shape: lanes per row L and chunks per lane V,
-// or false. H <= 8 heads, C a multiple of the 16-byte chunk width W with cq =
-// C/W a power of two (head sums and per-head dot products are butterflies
-// over lane bits); narrow rows (H*cq <= 64 chunks) take L = pow2ceil(H*cq),
-// V = 1; wide rows take L = 64 and V = H*cq/64 in {2, 3, 4, 6, 8} (cq <= 64
-// divides 64, so a lane's chunks share one channel chunk).
-inline bool fl_geom_w(int W, int H, int C, int& L, int& V) {
+// or false. H <= 8 heads, C a multiple of the 16-byte chunk width W; a head's
+// chunks are padded to cqp = pow2ceil(C/W) chunk slots (head sums and per-head
+// dot products are butterflies over lane bits). Narrow rows (H*cqp <= 64
+// slots) take L = pow2ceil(H*cqp), V = 1; wide rows take L = 64 and V in {2, 3,
+// 4, 6, 8} (cqp <= 64 divides 64, so a lane's chunks share one channel
+// chunk). `exact`: no slot is padding but those past a narrow row's heads.
+inline bool fl_geom_w(int W, int H, int C, int& L, int& V, bool& exact) {
+  if (H < 1 || H > kFlHeads || C < W || C % W != 0) return false;
   const int cq = C / W;
-  if (H < 1 || H > kFlHeads || C % W != 0 || cq < 1 || (cq & (cq - 1)) != 0) return false;
-  const int nq = H * cq;
+  const int cqp = pow2ceil(cq);
+  const int nq = H * cqp;
+  exact = cqp == cq;
   if (nq <= kWave) {
-    L = 1;
-    while (L < nq) L <<= 1;
+    L = pow2ceil(nq);
     V = 1;
     return true;
   }
-  if (cq > kWave || nq % kWave != 0) return false;
+  if (cqp > kWave) return false;
   L = kWave;
-  V = nq / kWave;
-  return V == 2 || V == 3 || V == 4 || V == 6 || V == 8;
+  V = (nq + kWave - 1) / kWave;
+  if (V == 5 || V == 7) ++V;
+  exact = exact && V * kWave == nq;
+  return true;
 }
 
-inline bool fl_geom(int dtype, int H, int C, int& L, int& V) {
-  return fl_geom_w(dtype == kBF16 || dtype == kBF16F32 ? 8 : 4, H, C, L, V);
+// Shapes that save and read per-row aggregates, that take dtype 2 and that
+// can be sharded: the exact ones.
+inline bool fl_exact(int dtype, int H, int C) {
+  int L, V;
+  bool exact;
+  return fl_geom_w(dtype == kBF16 || dtype == kBF16F32 ? 8 : 4, H, C, L, V, exact) && exact;
 }
 
+// Shapes the feature-layout kernels run.
 inline bool fl_ok(int dtype, int H, int C) {
   int L, V;
-  return fl_geom(dtype, H, C, L, V);
+  bool exact;
+  return fl_geom_w(dtype == kBF16 || dtype == kBF16F32 ? 8 : 4, H, C, L, V, exact) &&
+         (exact || dtype != kBF16F32);
 }
 
 // Whether bf16 features run the feature-layout kernels four values per lane
@@ -126,7 +137,8 @@ inline bool fl_ok(int dtype, int H, int C) {
 // dependent memory rounds is bound by.
 inline bool fl_half(int dtype, int H, int C, int64_t graph_nnz) {
   int L, V;
-  return dtype == kBF16 && graph_nnz < big_graph_edges() && fl_ok(dtype, H, C) && fl_geom_w(4, H, C, L, V) &&
+  bool exact;
+  return dtype == kBF16 && graph_nnz < big_graph_edges() && fl_ok(dtype, H, C) && fl_geom_w(4, H, C, L, V, exact) &&
          V == 1;
 }
 
@@ -172,7 +184,7 @@ int fl_dispatch_narrow(int L, Go&& go) {
 
 inline int fl_lgcq_w(int W, int C) {
   int lg = 0;
-  while ((1 << lg) < C / W) ++lg;
+  while ((1 << lg) < C / W) ++lg;  // C / W chunks in 2^lg slots
   return lg;
 }
 
@@ -238,7 +250,7 @@ int64_t cign_gat_fwd_workspace_bytes(int32_t n_seg, int32_t heads, int32_t chann
 // Floats of the per-row aggregate buffer of cign_gat_fwd / cign_gat_bwd for
 // this shape, 0 when the shape's kernels do not use one.
 int64_t cign_gat_row_agg_floats(int32_t dtype, int32_t n, int32_t heads, int32_t channels) {
-  if (n < 0 || heads < 1 || channels < 1 || !fl_ok(dtype, heads, channels)) return 0;
+  if (n < 0 || heads < 1 || channels < 1 || !fl_exact(dtype, heads, channels)) return 0;
   return static_cast<int64_t>(n) * heads * (2LL * channels + 1);
 }
 
@@ -282,8 +294,9 @@ int gat_fwd_impl(void* stream, int32_t dtype, int32_t n, int32_t nnz, int32_t he
     a.mask = edge_mask; a.partial = static_cast<float*>(workspace); a.counters = row_counters;
     a.agg = row_agg;
     int L, V;
-    if (fl_geom_w(FlGeom<T>::W, heads, channels, L, V)) {
-      if (!aligned16(xt) || !aligned16(ot) || !aligned16(pre))
+    bool exact;
+    if (fl_geom_w(FlGeom<T>::W, heads, channels, L, V, exact) && (exact || !std::is_same_v<T, bf16x>)) {
+      if (exact && (!aligned16(xt) || !aligned16(ot) || !aligned16(pre)))
         return set_error(kInvalid, "cign_gat_fwd: in_feat, out and pre must be 16-byte aligned");
       const int lgcq = fl_lgcq_w(FlGeom<T>::W, channels);
       auto go = [&](auto LC, auto VC) {
@@ -402,8 +415,10 @@ int gat_bwd_impl(void* stream, int32_t dtype, int32_t n, int32_t nnz, int32_t he
     a.row_counters = row_counters; a.col_counters = col_counters;
     a.grad_feat = gxt; a.grad_attn_row = grad_attn_row; a.grad_attn_col = grad_attn_col; a.grad_bias = grad_bias;
     int FL, FV;
-    if (fl_geom_w(FlGeom<T>::W, heads, channels, FL, FV)) {
-      if (!aligned16(xt) || !aligned16(gyt) || !aligned16(gxt) || !aligned16(pre) || !aligned16(grad_bias))
+    bool exact;
+    if (fl_geom_w(FlGeom<T>::W, heads, channels, FL, FV, exact) && (exact || !std::is_same_v<T, bf16x>)) {
+      if (exact &&
+          (!aligned16(xt) || !aligned16(gyt) || !aligned16(gxt) || !aligned16(pre) || !aligned16(grad_bias)))
         return set_error(kInvalid, "cign_gat_bwd: in_feat, pre, grad_y, grad_feat and grad_bias must be 16-byte "
                                    "aligned");
       // one contiguous record per destination row: g_pre, then H float4s

@@ -1,16 +1,26 @@
 // Collapsed GAT, feature layout: the gfx950 fast path for H <= 8 heads and C
-// a multiple of the 16-byte chunk width W (4 fp32 or 8 bf16 values) with
-// cq = C/W a power of two, and either H*cq <= 64 chunks (narrow rows) or cq <=
-// 64 with V = H*cq/64 in {2, 3, 4, 6, 8} chunks per lane (wide rows, e.g. the
-// production H=6 x C=256). Semantics are those stated at the top of
-// gat_kernels.h (reference collapsed_gat_cuda.cu:34-430).
+// a multiple of the 16-byte chunk width W (4 fp32 or 8 bf16 values). A head's
+// C/W chunks sit in cq = pow2ceil(C/W) chunk slots; rows of at most 64 slots
+// are narrow, wider ones take V = ceil(H*cq/64) in {2, 3, 4, 6, 8} slots per
+// lane (5 and 7 run as 6 and 8; e.g. the production H=6 x C=256). Semantics
+// are those stated at the top of gat_kernels.h (reference
+// collapsed_gat_cuda.cu:34-430).
+//
+// A slot without a chunk (C/W no power of two, or V*64 > H*cq) repeats a load
+// of its head and adds nothing to sums or outputs. Such shapes ran the pair
+// layout (gat_kernels.h) before, whose lane reads one (edge, head)'s whole
+// run of channels, 64 different runs per load: forward / backward, fp32,
+// 10,007 nodes x 5 x 48 101 / 101 -> 25 / 51 us, 24,492 nodes x 3 x 100 344 /
+// 351 -> 46 / 84, 8 x 192 766 / 862 -> 183 / 276, 5 x 256 926 / 953 -> 152 /
+// 230; bf16 6 x 96 366 / 394 -> 61 / 108. It keeps H > 8 and channels that
+// are no multiple of W.
 //
 // Geometry (shared with the SpMM, schedule.h built with light_max = 64 and a
 // segment length that is a multiple of 256). A group of L lanes owns one row;
-// lane gl owns the V chunks q = v*L + gl (v < V) of a feature row, chunk q
+// lane gl owns the V chunk slots q = v*L + gl (v < V) of a feature row, slot q
 // being head hq = q / cq, channel chunk cw = q % cq. Narrow rows have V = 1
 // and L = pow2ceil(H*cq); wide rows have L = 64 and, as cq divides 64, every
-// chunk of a lane has the same channel chunk cw = gl % cq and its own head.
+// slot of a lane has the same channel chunk cw = gl % cq and its own head.
 // Rows with degree <= L go one per group (64/L rows per wavefront), rows
 // with degree <= 64 one per wavefront (its groups split the edges), heavier
 // rows are segments (one 4-wave workgroup each, rounds of 256 edges) whose
@@ -101,6 +111,10 @@ constexpr int kFwdUBig = CIGN_FL_FWD_U_BIG;
 // keep 16.
 constexpr int kFwdUNarrowF32 = 8;
 constexpr int kRowsU = CIGN_FL_ROWS_U;
+// Rows of 8-value (bf16) chunks: half of it. 6 x 256 (three chunks a lane),
+// 211K edges: the rows pass 101 us with 4 slots (233 VGPRs), 93 with 2; 4-value
+// chunks keep the larger batch (5 x 96: 38 us against 48).
+constexpr int kRowsUWide = CIGN_FL_ROWS_U / 2;
 constexpr int kColsU = CIGN_FL_COLS_U;
 // Batch cap of the shared-weight columns batches (large graphs): 4 slots
 // measured 3.54 ms at 62.4M edges against 3.90 ms for 8 and 5.55 ms for 16.
@@ -136,33 +150,50 @@ struct FlGeom<bf16h> {
 };
 
 // Lane geometry of a group of L lanes (one row) owning V chunks per lane.
+// Chunk slot qq = v * L + gl is head qq >> lgcq, channel chunk qq & (2^lgcq -
+// 1); slots past the heads, or past the C / W chunks of a padded head, own
+// nothing (qv false) and read a chunk that is there. hv: the slot's head is
+// one of the heads (its lane shares in that head's per-edge work even where
+// it owns no chunk).
 template <int L, int V>
 struct FlLane {
   static_assert(V == 1 || L == kWave, "several chunks per lane need a full wavefront per row");
   int lane, g, gl, cw;
-  int q[V], hq[V];
-  bool qv[V];
-  __device__ __forceinline__ FlLane(int lgcq, int nq) {
+  int off[V], hq[V];
+  bool qv[V], hv[V];
+  __device__ __forceinline__ FlLane(int lgcq, int H, int C, int W) {
     lane = lane_id();
     g = lane / L;
     gl = lane & (L - 1);
+    const int slot = gl & ((1 << lgcq) - 1);  // the same for every v: 2^lgcq divides L where V > 1
+    const int last = C / W - 1;
+    cw = min(slot, last);
 #pragma unroll
     for (int v = 0; v < V; ++v) {
-      const int qq = v * L + gl;
-      qv[v] = qq < nq;
-      q[v] = qv[v] ? qq : 0;
-      hq[v] = q[v] >> lgcq;
+      const int h = (v * L + gl) >> lgcq;
+      hv[v] = h < H;
+      qv[v] = hv[v] && slot <= last;
+      hq[v] = hv[v] ? h : 0;
+      off[v] = hq[v] * C + cw * W;
     }
-    cw = V == 1 ? (q[0] & ((1 << lgcq) - 1)) : (gl & ((1 << lgcq) - 1));
   }
 };
 
-// W fp32 values from a 16-byte aligned address.
+// Raw chunk at p, in one access whatever p's alignment.
+template <typename T, int W>
+__device__ __forceinline__ typename Chunk<T, W>::Raw load_chunk(const T* p) {
+  typename Chunk<T, W>::Raw r;
+  __builtin_memcpy(&r, p, sizeof(r));
+  return r;
+}
+
+// W fp32 values, four (16 bytes) an access whatever p's alignment.
 template <int W>
 __device__ __forceinline__ void load_f32(const float* p, float (&v)[W]) {
 #pragma unroll
   for (int k = 0; k < W; k += 4) {
-    const float4 t = *reinterpret_cast<const float4*>(p + k);
+    float4 t;
+    __builtin_memcpy(&t, p + k, sizeof(t));
     v[k] = t.x;
     v[k + 1] = t.y;
     v[k + 2] = t.z;
@@ -173,7 +204,29 @@ __device__ __forceinline__ void load_f32(const float* p, float (&v)[W]) {
 template <int W>
 __device__ __forceinline__ void store_f32(float* p, const float (&v)[W]) {
 #pragma unroll
-  for (int k = 0; k < W; k += 4) *reinterpret_cast<float4*>(p + k) = make_float4(v[k], v[k + 1], v[k + 2], v[k + 3]);
+  for (int k = 0; k < W; k += 4) {
+    const float4 t = make_float4(v[k], v[k + 1], v[k + 2], v[k + 3]);
+    __builtin_memcpy(p + k, &t, sizeof(t));
+  }
+}
+
+// W outputs (or incoming gradients) of type T as fp32.
+template <typename T, int W>
+__device__ __forceinline__ void load_values(const T* p, float (&v)[W]) {
+  if constexpr (std::is_same_v<T, float>) load_f32<W>(p, v);
+  else Chunk<T, W>::unpack(load_chunk<T, W>(p), v);
+}
+template <typename T, int W>
+__device__ __forceinline__ void store_values(T* p, const float (&v)[W]) {
+  if constexpr (std::is_same_v<T, float>) {
+    store_f32<W>(p, v);
+  } else {
+    uint32_t w[W / 2];
+#pragma unroll
+    for (int k = 0; k < W / 2; ++k)
+      w[k] = from_f32<bf16>(v[2 * k]).bits | (static_cast<uint32_t>(from_f32<bf16>(v[2 * k + 1]).bits) << 16);
+    __builtin_memcpy(p, w, sizeof(w));
+  }
 }
 
 // Largest value of v over the groups of a wavefront (lane bits >= log2 L).
@@ -354,8 +407,8 @@ struct FwdBatches {
       const uint64_t j = static_cast<uint32_t>(shfl(jj, (ub + k * step) & (kWave - 1)));
 #pragma unroll
       for (int v = 0; v < V; ++v)
-        xb[k][v] = *reinterpret_cast<const typename Chunk<T, W>::Raw*>(
-            reinterpret_cast<const char*>(a.x + ln.q[v] * W) + j * rowB);
+        xb[k][v] = load_chunk<T, W>(
+            reinterpret_cast<const T*>(reinterpret_cast<const char*>(a.x + ln.off[v]) + j * rowB));
     }
     const int r = ln.gl & (R - 1);
     float sc[NT][V];
@@ -390,7 +443,7 @@ struct FwdBatches {
         if constexpr (DROP) {
           const int64_t idx = static_cast<int64_t>(ebase + uo[t]) * a.H + ln.hq[v];
           const bool keep = gat_keep(a.seed, static_cast<uint64_t>(idx + a.mask_base), a.p);
-          if (own[t] && ln.qv[v]) a.mask[idx] = keep ? 1 : 0;
+          if (own[t] && ln.hv[v]) a.mask[idx] = keep ? 1 : 0;
           w = keep ? pk * (1.0f / (1.0f - a.p)) : 0.0f;
         }
         wk[t][v] = w;
@@ -488,8 +541,8 @@ __device__ __forceinline__ void fwd_emit(const GatFwdArgs<T>& a, const FlLane<L,
       float yl[W];
 #pragma unroll
       for (int w = 0; w < W; ++w) yl[w] = st.accl[v][w] * inv;
-      store_f32<W>(a.agg + static_cast<int64_t>(row) * F + ln.q[v] * W, yv);
-      store_f32<W>(a.agg + nF + static_cast<int64_t>(row) * F + ln.q[v] * W, yl);
+      store_f32<W>(a.agg + static_cast<int64_t>(row) * F + ln.off[v], yv);
+      store_f32<W>(a.agg + nF + static_cast<int64_t>(row) * F + ln.off[v], yl);
       if (ln.cw == 0) a.agg[2 * nF + static_cast<int64_t>(row) * a.H + ln.hq[v]] = st.bl[v] * inv;
     }
   }
@@ -510,7 +563,7 @@ __device__ __forceinline__ void fwd_emit(const GatFwdArgs<T>& a, const FlLane<L,
       o[w] = silu(pr[w]);
     }
     store_f32<W>(a.pre + base, pr);
-    Chunk<GatOut<T>, W>::store(a.out + base, o);
+    store_values<GatOut<T>, W>(a.out + base, o);
   }
   if (ln.cw == 0)
 #pragma unroll
@@ -563,9 +616,8 @@ __global__ __launch_bounds__(kBlock) void gat_fwd_fl_kernel(GatFwdArgs<T> a, Sch
   constexpr int W = FlGeom<T>::W;
   constexpr int G = kWave / L;
   const int cq = 1 << lgcq;
-  const int nq = a.H * cq;
   const int F = a.H * a.C;
-  const FlLane<L, V> ln(lgcq, nq);
+  const FlLane<L, V> ln(lgcq, a.H, a.C, W);
   const int wave = wave_id();
   FwdState<W, V> st;
   st.clear();
@@ -636,8 +688,8 @@ __global__ __launch_bounds__(kBlock) void gat_fwd_fl_kernel(GatFwdArgs<T> a, Sch
 #pragma unroll
     for (int v = 0; v < V; ++v)
       if (ln.qv[v]) {
-        st_agent_n<W>(mine + ln.q[v] * W, st.acc[v]);
-        st_agent_n<W>(mine + F + ln.q[v] * W, st.accl[v]);
+        st_agent_n<W>(mine + ln.off[v], st.acc[v]);
+        st_agent_n<W>(mine + F + ln.off[v], st.accl[v]);
         if (ln.cw == 0) {
           st_agent(mine + 2 * F + ln.hq[v], st.m[v]);
           st_agent(mine + 2 * F + a.H + ln.hq[v], st.s[v]);
@@ -653,8 +705,8 @@ __global__ __launch_bounds__(kBlock) void gat_fwd_fl_kernel(GatFwdArgs<T> a, Sch
 #pragma unroll
     for (int v = 0; v < V; ++v) {
       float a2[W], l2[W];
-      ld_agent_n<W>(pz + ln.q[v] * W, a2);
-      ld_agent_n<W>(pz + F + ln.q[v] * W, l2);
+      ld_agent_n<W>(pz + ln.off[v], a2);
+      ld_agent_n<W>(pz + F + ln.off[v], l2);
       st.merge(v, ld_agent(pz + 2 * F + ln.hq[v]), ld_agent(pz + 2 * F + a.H + ln.hq[v]),
                ld_agent(pz + 2 * F + 2 * a.H + ln.hq[v]), a2, l2);
     }
@@ -774,7 +826,7 @@ struct RowBatches {
 #pragma unroll
       for (int v = 0; v < V; ++v) {
         ab[k][v] = a.attn_col[static_cast<int64_t>(j) * a.H + ln.hq[v]];
-        xb[k][v] = Chunk<T, W>::load_raw(a.x + static_cast<int64_t>(j) * F + ln.q[v] * W);
+        xb[k][v] = load_chunk<T, W>(a.x + static_cast<int64_t>(j) * F + ln.off[v]);
       }
     }
     // Dropout mask bytes: each (edge, head) pair loaded once.
@@ -813,7 +865,7 @@ __device__ __forceinline__ void rows_edges(const GatBwdArgs<T>& a, const FlLane<
                                            int first, int step, int cnt, int need, int ebase, const RowHead<V>& rh,
                                            RowAcc<FlGeom<T>::W, V>& st) {
   RowBatches<T, L, V, DROP> rb{a, ln, jj, base, first, step, cnt, ebase, rh, st};
-  for_batches<batch_cap(kRowsU, V)>(need, rb);
+  for_batches<batch_cap(FlGeom<T>::W == 8 ? kRowsUWide : kRowsU, V)>(need, rb);
 }
 
 template <int L, int W, int V>
@@ -833,17 +885,24 @@ __device__ __forceinline__ void grad_pre_chunk(const GatBwdArgs<T>& a, int row, 
   constexpr int W = FlGeom<T>::W;
   const int64_t base = static_cast<int64_t>(row) * a.C + cw * W;
   float gy[W], pr[W];
-  Chunk<GatOut<T>, W>::load(a.grad_y + base, gy);
+  load_values<GatOut<T>, W>(a.grad_y + base, gy);
   load_f32<W>(a.pre + base, pr);
 #pragma unroll
   for (int w = 0; w < W; ++w) gp[w] = gy[w] * silu_grad(pr[w]);
 }
 
-// (wsum, A) of each of the lane's heads from the accumulated chunks: dot with
-// g_pre, summed over the head's cq lanes, divided by H.
-template <int W, int V>
-__device__ __forceinline__ void rows_dots(const RowAcc<W, V>& st, const float (&gp)[W], int cq, float inv_h,
-                                          float (&wsum)[V], float (&A)[V]) {
+// Of each of the lane's heads, from the accumulated chunks: wsum = <g_pre,
+// vs> / H and A = <g_pre, vsl - B vs> / H, summed over the head's chunk slots.
+// With the row's whole B that A is grad_attn_row: the two feature sums cancel
+// channel by channel before the dot product, not the two dot products after
+// it (5 x 48 channels, against 64 bits: 4e-7 -> 3e-7). With B = 0 it is the
+// plain dot product, for parts of a heavy row, and for the rows of the
+// aggregate kernel, a stream whose registers that B costs (6 x 256 bf16: 62 ->
+// 76 VGPRs, 8 -> 6 wavefronts per SIMD, the backward 144 -> 150 us).
+template <int L, int W, int V>
+__device__ __forceinline__ void rows_dots(const FlLane<L, V>& ln, const RowAcc<W, V>& st, const float (&B)[V],
+                                          const float (&gp)[W], int cq, float inv_h, float (&wsum)[V],
+                                          float (&A)[V]) {
   float d[2 * V];
 #pragma unroll
   for (int v = 0; v < V; ++v) {
@@ -851,10 +910,10 @@ __device__ __forceinline__ void rows_dots(const RowAcc<W, V>& st, const float (&
 #pragma unroll
     for (int w = 0; w < W; ++w) {
       d1 = fmaf(gp[w], st.vs[v][w], d1);
-      d2 = fmaf(gp[w], st.vsl[v][w], d2);
+      d2 = fmaf(gp[w], fmaf(-B[v], st.vs[v][w], st.vsl[v][w]), d2);
     }
-    d[v] = d1;
-    d[V + v] = d2;
+    d[v] = ln.qv[v] ? d1 : 0.0f;
+    d[V + v] = ln.qv[v] ? d2 : 0.0f;
   }
   head_sum_n<2 * V>(d, cq);
 #pragma unroll
@@ -866,8 +925,8 @@ __device__ __forceinline__ void rows_dots(const RowAcc<W, V>& st, const float (&
 
 template <typename T>
 __device__ __forceinline__ void rows_store(const GatBwdArgs<T>& a, int row, int hq, float ar, float em, float ies,
-                                           float wsum, float A, float B) {
-  a.grad_attn_row[static_cast<int64_t>(row) * a.H + hq] = A - wsum * B;
+                                           float wsum, float grad) {
+  a.grad_attn_row[static_cast<int64_t>(row) * a.H + hq] = grad;
   a.rowstat[static_cast<int64_t>(row) * a.rs_stride + hq] = make_float4(ar, em, ies, wsum);
 }
 
@@ -875,13 +934,13 @@ __device__ __forceinline__ void rows_store(const GatBwdArgs<T>& a, int row, int 
 // (lanes cw = 0) and the g_pre chunk (head-0 lanes).
 template <typename T, int L, int V>
 __device__ __forceinline__ void rows_emit(const GatBwdArgs<T>& a, const FlLane<L, V>& ln, int row,
-                                          const RowHead<V>& rh, const float (&wsum)[V], const float (&A)[V],
-                                          const float (&B)[V], const float (&gp)[FlGeom<T>::W]) {
+                                          const RowHead<V>& rh, const float (&wsum)[V], const float (&grad)[V],
+                                          const float (&gp)[FlGeom<T>::W]) {
   constexpr int W = FlGeom<T>::W;
   if (ln.cw == 0)
 #pragma unroll
     for (int v = 0; v < V; ++v)
-      if (ln.qv[v]) rows_store(a, row, ln.hq[v], rh.ar[v], rh.em[v], rh.ies[v], wsum[v], A[v], B[v]);
+      if (ln.qv[v]) rows_store(a, row, ln.hq[v], rh.ar[v], rh.em[v], rh.ies[v], wsum[v], grad[v]);
   if (ln.qv[0] && ln.hq[0] == 0) store_f32<W>(a.grad_pre + static_cast<int64_t>(row) * a.gp_stride + ln.cw * W, gp);
 }
 
@@ -891,8 +950,7 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_rows_fl_kernel(GatBwdArgs<T> a
   constexpr int W = FlGeom<T>::W;
   constexpr int G = kWave / L;
   const int cq = 1 << lgcq;
-  const int nq = a.H * cq;
-  const FlLane<L, V> ln(lgcq, nq);
+  const FlLane<L, V> ln(lgcq, a.H, a.C, W);
   const int wave = wave_id();
   __shared__ float red[kWavesPerBlock][3][kFlHeads];
   __shared__ int flag;
@@ -928,8 +986,8 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_rows_fl_kernel(GatBwdArgs<T> a
       rows_edges<T, L, V, DROP>(a, ln, jj, 0, ln.g, G, deg, (deg + G - 1) / G, r.y, rh, st);
       rows_group_sum<L, W, V>(st);
     }
-    rows_dots<W, V>(st, gp, cq, a.inv_h, wsum, A);
-    if (has && (tiny || ln.g == 0)) rows_emit(a, ln, row, rh, wsum, A, st.B, gp);
+    rows_dots<L, W, V>(ln, st, st.B, gp, cq, a.inv_h, wsum, A);
+    if (has && (tiny || ln.g == 0)) rows_emit(a, ln, row, rh, wsum, A, gp);
     return;
   }
 
@@ -951,7 +1009,8 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_rows_fl_kernel(GatBwdArgs<T> a
     jj = jn;
   }
   rows_group_sum<L, W, V>(st);
-  rows_dots<W, V>(st, gp, cq, a.inv_h, wsum, A);
+  const float none[V] = {};
+  rows_dots<L, W, V>(ln, st, none, gp, cq, a.inv_h, wsum, A);
   if (ln.g == 0 && ln.cw == 0)
 #pragma unroll
     for (int v = 0; v < V; ++v)
@@ -974,7 +1033,7 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_rows_fl_kernel(GatBwdArgs<T> a
       const int h = threadIdx.x;
       float ar, em, ies;
       row_head1(a, row, h, ar, em, ies);
-      rows_store(a, row, h, ar, em, ies, red[0][0][h], red[0][1][h], red[0][2][h]);
+      rows_store(a, row, h, ar, em, ies, red[0][0][h], red[0][1][h] - red[0][0][h] * red[0][2][h]);
     }
     return;
   }
@@ -992,7 +1051,7 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_rows_fl_kernel(GatBwdArgs<T> a
     }
     float ar, em, ies;
     row_head1(a, row, h, ar, em, ies);
-    rows_store(a, row, h, ar, em, ies, w, AA, BB);
+    rows_store(a, row, h, ar, em, ies, w, AA - w * BB);
   }
 }
 
@@ -1004,7 +1063,7 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_rows_agg_kernel(GatBwdArgs<T> 
   constexpr int W = FlGeom<T>::W;
   constexpr int G = kWave / L;
   const int cq = 1 << lgcq;
-  const FlLane<L, V> ln(lgcq, a.H * cq);
+  const FlLane<L, V> ln(lgcq, a.H, a.C, W);
   const int row = (blockIdx.x * kWavesPerBlock + wave_id()) * G + ln.g;
   if (row >= a.n) return;  // no barrier follows
   const int F = a.H * a.C;
@@ -1012,16 +1071,19 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_rows_agg_kernel(GatBwdArgs<T> 
   RowAcc<W, V> st;
 #pragma unroll
   for (int v = 0; v < V; ++v) {
-    load_f32<W>(a.agg + static_cast<int64_t>(row) * F + ln.q[v] * W, st.vs[v]);
-    load_f32<W>(a.agg + nF + static_cast<int64_t>(row) * F + ln.q[v] * W, st.vsl[v]);
+    load_f32<W>(a.agg + static_cast<int64_t>(row) * F + ln.off[v], st.vs[v]);
+    load_f32<W>(a.agg + nF + static_cast<int64_t>(row) * F + ln.off[v], st.vsl[v]);
     st.B[v] = a.agg[2 * nF + static_cast<int64_t>(row) * a.H + ln.hq[v]];
   }
   float gp[W];
   grad_pre_chunk(a, row, ln.cw, gp);
   const RowHead<V> rh = row_head(a, row, ln);  // issued with the loads above, before any use
   float wsum[V], A[V];
-  rows_dots<W, V>(st, gp, cq, a.inv_h, wsum, A);
-  rows_emit(a, ln, row, rh, wsum, A, st.B, gp);
+  const float none[V] = {};
+  rows_dots<L, W, V>(ln, st, none, gp, cq, a.inv_h, wsum, A);
+#pragma unroll
+  for (int v = 0; v < V; ++v) A[v] -= wsum[v] * st.B[v];
+  rows_emit(a, ln, row, rh, wsum, A, gp);
 }
 
 // ===========================================================================
@@ -1333,13 +1395,13 @@ struct XCol {
   __device__ __forceinline__ void prefetch(const GatBwdArgs<T>& a, const FlLane<L, V>& ln, int j) {
     if constexpr (kEarly)
 #pragma unroll
-      for (int v = 0; v < V; ++v) raw[v] = Chunk<T, W>::load_raw(a.x + static_cast<int64_t>(j) * a.H * a.C + ln.q[v] * W);
+      for (int v = 0; v < V; ++v) raw[v] = load_chunk<T, W>(a.x + static_cast<int64_t>(j) * a.H * a.C + ln.off[v]);
   }
   template <int L>
   __device__ __forceinline__ void get(const GatBwdArgs<T>& a, const FlLane<L, V>& ln, int j, int v,
                                       float (&xj)[W]) const {
     if constexpr (kEarly) Chunk<T, W>::unpack(raw[v], xj);
-    else Chunk<T, W>::load(a.x + static_cast<int64_t>(j) * a.H * a.C + ln.q[v] * W, xj);
+    else Chunk<T, W>::unpack(load_chunk<T, W>(a.x + static_cast<int64_t>(j) * a.H * a.C + ln.off[v]), xj);
   }
 };
 
@@ -1357,6 +1419,7 @@ __device__ __forceinline__ void cols_gac(const GatBwdArgs<T>& a, const FlLane<L,
     d[v] = 0.0f;
 #pragma unroll
     for (int w = 0; w < W; ++w) d[v] = fmaf(st.ua[v][w], xj[w], d[v]);
+    d[v] = ln.qv[v] ? d[v] : 0.0f;
   }
   head_sum_n<V>(d, cq);
 #pragma unroll
@@ -1382,9 +1445,8 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_cols_fl_kernel(GatBwdArgs<T> a
   constexpr int W = FlGeom<T>::W;
   constexpr int G = kWave / L;
   const int cq = 1 << lgcq;
-  const int nq = a.H * cq;
   const int F = a.H * a.C;
-  const FlLane<L, V> ln(lgcq, nq);
+  const FlLane<L, V> ln(lgcq, a.H, a.C, W);
   const int wave = wave_id();
   __shared__ float red[V * kWave * W];
   __shared__ float gred[kWavesPerBlock][kFlHeads];
@@ -1442,7 +1504,7 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_cols_fl_kernel(GatBwdArgs<T> a
       float o[W];
 #pragma unroll
       for (int w = 0; w < W; ++w) o[w] = st.ug[v][w] * a.inv_h;
-      Chunk<GatOut<T>, W>::store(a.grad_feat + static_cast<int64_t>(j) * F + ln.q[v] * W, o);
+      store_values<GatOut<T>, W>(a.grad_feat + static_cast<int64_t>(j) * F + ln.off[v], o);
       if (ln.cw == 0) a.grad_attn_col[static_cast<int64_t>(j) * a.H + ln.hq[v]] = gac[v];
     }
     return;
@@ -1485,7 +1547,7 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_cols_fl_kernel(GatBwdArgs<T> a
         if (ln.qv[v])
 #pragma unroll
           for (int w = 0; w < W; ++w) {
-            float& d = red[ln.q[v] * W + w];
+            float& d = red[ln.off[v] + w];
             d = src == 0 ? st.ug[v][w] : d + st.ug[v][w];
           }
     __syncthreads();

@@ -370,3 +370,57 @@ def test_wide_rows_long_segments(H, C, dtype, p, agg_mode, monkeypatch):
     assert_close(gac.cpu().numpy(), gr["grad_attn_col"], name="grad_attn_col", **tol)
     assert_close(gb.cpu().numpy(), gr["grad_bias"], name="grad_bias", **tol)
     S._CACHE.clear()
+
+
+# Heads padded to a power of two of chunk slots: 12 -> 16, 25 -> 32 and 3 -> 4
+# chunks (a quad with a lane that owns nothing, with dropout), rows that end
+# inside a wavefront's slots (5 and 7 x 64 chunks in 6 and 8 per lane), the
+# narrowest and the widest, bf16 rows whose small-graph lanes hold four values.
+PADDED = [
+    (5, 48, 0.0, torch.float32, 400, {0: 700, 2: 260}),
+    (3, 100, 0.2, torch.float32, 300, {1: 520}),
+    (4, 12, 0.3, torch.float32, 300, {1: 600, 9: 70}),
+    (1, 12, 0.25, torch.float32, 200, {}),
+    (8, 20, 0.0, torch.float32, 300, {3: 300}),
+    (5, 256, 0.1, torch.float32, 200, {2: 600}),
+    (7, 256, 0.0, torch.float32, 150, {0: 300}),
+    (8, 252, 0.0, torch.float32, 120, {4: 300}),
+    (5, 96, 0.2, torch.bfloat16, 300, {0: 600}),
+    (2, 24, 0.3, torch.bfloat16, 300, {1: 700}),
+    (7, 248, 0.0, torch.bfloat16, 150, {1: 400}),
+]
+
+
+@pytest.mark.parametrize("big", [False, True], ids=["small-graph-kernels", "large-graph-kernels"])
+@pytest.mark.parametrize("H,C,p,dtype,n,hubs", PADDED)
+def test_padded_heads_match_oracle(H, C, p, dtype, n, hubs, big, monkeypatch):
+    test_ext_forward_backward_matches_oracle(H, C, p, dtype, n, hubs, True, big, monkeypatch)
+
+
+@pytest.mark.parametrize("H,C,dtype", [(5, 48, torch.float32), (5, 24, torch.bfloat16)])
+def test_padded_heads_unaligned_tensors(H, C, dtype):
+    """Tensors that start off a 16-byte boundary (views into a buffer) give
+    the aligned tensors' results bit for bit on the padded shapes."""
+    from cign_amd.collapsed_gat import ensure_collapsed_gat_loaded
+
+    rng = np.random.default_rng(H * C)
+    n = 200
+    rowptr, col, row, colptr, perm = _dev_graph(_graph(rng, n, {0: 300}), n)
+    x, ar, ac, b, gy = _inputs(rng, n, H, C, dtype)
+
+    def shifted(t):
+        buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+        buf[1:] = t.reshape(-1)
+        v = buf[1:].view(t.shape)
+        assert v.data_ptr() % 16 != 0
+        return v
+
+    ext = ensure_collapsed_gat_loaded()
+    out, pre, emax, esum, mask = ext.forward(ar, ac, rowptr, col, 0.2, x, b, 0.0, 0)
+    grads = ext.backward(0.2, 0.0, rowptr, col, colptr, row, perm, emax, esum, mask, x, ar, ac, pre, gy)
+    out2 = ext.forward(ar, ac, rowptr, col, 0.2, shifted(x), shifted(b), 0.0, 0)[0]
+    grads2 = ext.backward(0.2, 0.0, rowptr, col, colptr, row, perm, emax, esum, mask, shifted(x), ar, ac, shifted(pre),
+                          shifted(gy))
+    assert torch.equal(out, out2)
+    for a, e in zip(grads2, grads):
+        assert torch.equal(a, e)
