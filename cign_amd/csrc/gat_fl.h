@@ -895,10 +895,11 @@ __device__ __forceinline__ void grad_pre_chunk(const GatBwdArgs<T>& a, int row, 
 // vs> / H and A = <g_pre, vsl - B vs> / H, summed over the head's chunk slots.
 // With the row's whole B that A is grad_attn_row: the two feature sums cancel
 // channel by channel before the dot product, not the two dot products after
-// it (5 x 48 channels, against 64 bits: 4e-7 -> 3e-7). With B = 0 it is the
-// plain dot product, for parts of a heavy row, and for the rows of the
-// aggregate kernel, a stream whose registers that B costs (6 x 256 bf16: 62 ->
-// 76 VGPRs, 8 -> 6 wavefronts per SIMD, the backward 144 -> 150 us).
+// it (fp32 4 x 16 and 5 x 48 channels, against 64 bits: 4e-7 -> 3e-7). With B
+// = 0 it is the plain dot product: for parts of a heavy row, and for 8-value
+// chunks in the aggregate kernel, a stream whose registers B costs there (6 x
+// 256 bf16: 62 -> 76 VGPRs, 8 -> 6 wavefronts per SIMD, the backward 144 ->
+// 150 us; 4-value chunks: fp32 6 x 256 171 us either way).
 template <int L, int W, int V>
 __device__ __forceinline__ void rows_dots(const FlLane<L, V>& ln, const RowAcc<W, V>& st, const float (&B)[V],
                                           const float (&gp)[W], int cq, float inv_h, float (&wsum)[V],
@@ -1079,10 +1080,14 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_rows_agg_kernel(GatBwdArgs<T> 
   grad_pre_chunk(a, row, ln.cw, gp);
   const RowHead<V> rh = row_head(a, row, ln);  // issued with the loads above, before any use
   float wsum[V], A[V];
-  const float none[V] = {};
-  rows_dots<L, W, V>(ln, st, none, gp, cq, a.inv_h, wsum, A);
+  if constexpr (W == 4) {
+    rows_dots<L, W, V>(ln, st, st.B, gp, cq, a.inv_h, wsum, A);
+  } else {
+    const float none[V] = {};
+    rows_dots<L, W, V>(ln, st, none, gp, cq, a.inv_h, wsum, A);
 #pragma unroll
-  for (int v = 0; v < V; ++v) A[v] -= wsum[v] * st.B[v];
+    for (int v = 0; v < V; ++v) A[v] -= wsum[v] * st.B[v];
+  }
   rows_emit(a, ln, row, rh, wsum, A, gp);
 }
 
