@@ -1,4 +1,5 @@
-"""Builds libcign_amd.so (gfx950 HIP kernels + C-ABI) in-tree with hipcc.
+"""Builds libcign_amd.so (gfx950 HIP kernels + C-ABI) in-tree with hipcc, and
+_cign.so, the CPython binding of its entry points.
 
 Run as ``python -m cign_amd._build`` or through ``__graft_entry__.build()``.
 Object files go to ``cign_amd/_build/`` and the library to
@@ -11,12 +12,15 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
 SRC = PKG / "csrc"
 OBJ = PKG / "_build"
 LIB = PKG / "libcign_amd.so"
+BINDING_SRC = SRC / "python" / "binding.cpp"
+BINDING = PKG / "_cign.so"
 
 ARCH = "gfx950"
 
@@ -71,6 +75,20 @@ def _compile(hipcc: str, src: Path, force: bool) -> Path:
     return obj
 
 
+def build_binding() -> Path:
+    """Compiles the CPython binding against the library (host code only)."""
+    tmp = BINDING.with_suffix(".so.tmp")
+    cxx = os.environ.get("CXX") or shutil.which("g++") or str(Path(_hipcc()).parent / "amdclang++")
+    cmd = [cxx, "-O2", "-fPIC", "-std=c++17", "-Wall", "-shared", f"-I{sysconfig.get_paths()['include']}",
+           f"-I{PKG.parent / 'include'}", str(BINDING_SRC), "-o", str(tmp), f"-L{PKG}", f"-l:{LIB.name}",
+           "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"binding build failed:\n{res.stderr[-6000:]}")
+    os.replace(tmp, BINDING)
+    return BINDING
+
+
 def build(verbose: bool = False, jobs: int | None = None, force: bool = True) -> Path:
     """Compiles every HIP source for gfx950 and links libcign_amd.so.
 
@@ -91,6 +109,7 @@ def build(verbose: bool = False, jobs: int | None = None, force: bool = True) ->
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr[-6000:]}")
     os.replace(tmp, LIB)
+    build_binding()
     if verbose:
         print(f"built {LIB} from {len(srcs)} sources", flush=True)
     return LIB

@@ -1,4 +1,10 @@
-"""ctypes binding of libcign_amd.so, the C-ABI declared in include/cign_amd.h.
+"""Binding of libcign_amd.so, the C-ABI declared in include/cign_amd.h.
+
+The library's functions are reachable through ctypes as attributes of the
+object load_library() returns; ``call`` and the size functions go through
+_cign.so, a CPython module over the same library (csrc/python/binding.cpp),
+whose argument conversions cost a small part of ctypes' (a call with 30
+arguments: 3 us).
 
 The library is loaded after ``import torch`` so that it binds to the HIP
 runtime torch already loaded (same soname, one runtime per process). Every
@@ -96,19 +102,27 @@ _SIGNATURES = {
 _LOCK = threading.Lock()
 _LIB = None
 _LIB_ERROR: BaseException | None = None
+_GPU_SEEN = False
+
+
+# Entry points whose Python callers pass ctypes references (host outputs).
+_BY_REFERENCE = ("cign_row_schedule_size", "cign_gat_schedule_params")
 
 
 class _Lib:
-    def __init__(self, handle: C.CDLL):
+    def __init__(self, handle: C.CDLL, native):
         self._h = handle
+        self._fn = {}
         for name, (res, args) in _SIGNATURES.items():
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
-            setattr(self, name, fn)
+            self._fn[name] = fn if name in _BY_REFERENCE else getattr(native, name, fn)
+            sizes = name.endswith(("_bytes", "_floats"))
+            setattr(self, name, self._fn[name] if sizes else fn)
 
     def call(self, name: str, *args) -> None:
-        rc = getattr(self, name)(*args)
+        rc = self._fn[name](*args)
         if rc != 0:
             msg = self.cign_last_error().decode(errors="replace")
             raise RuntimeError(f"{name} failed (status {rc}): {msg}")
@@ -117,7 +131,9 @@ class _Lib:
 def load_library(require_gpu: bool = True) -> _Lib:
     """Loads libcign_amd.so once. Raises RuntimeError if it is not built or,
     when ``require_gpu``, if no HIP device is visible."""
-    global _LIB, _LIB_ERROR
+    global _LIB, _LIB_ERROR, _GPU_SEEN
+    if _GPU_SEEN:  # loaded, and a GPU was visible
+        return _LIB
     with _LOCK:
         if _LIB is None:
             if _LIB_ERROR is not None:
@@ -127,12 +143,20 @@ def load_library(require_gpu: bool = True) -> _Lib:
                     raise RuntimeError(
                         f"{LIB_PATH} is not built; run `python -m cign_amd._build` (hipcc, gfx950)"
                     )
-                _LIB = _Lib(C.CDLL(str(LIB_PATH)))
+                handle = C.CDLL(str(LIB_PATH))
+                try:
+                    from . import _cign
+                except ImportError as exc:
+                    raise RuntimeError(f"{LIB_PATH.with_name('_cign.so')} is not built; run "
+                                       "`python -m cign_amd._build`") from exc
+                _LIB = _Lib(handle, _cign)
             except BaseException as exc:  # cached and re-raised, like the reference loaders
                 _LIB_ERROR = exc
                 raise
-    if require_gpu and not torch.cuda.is_available():
-        raise RuntimeError("libcign_amd kernels require a HIP GPU (torch.cuda.is_available() is False)")
+    if require_gpu:
+        if not torch.cuda.is_available():
+            raise RuntimeError("libcign_amd kernels require a HIP GPU (torch.cuda.is_available() is False)")
+        _GPU_SEEN = True
     return _LIB
 
 
@@ -158,9 +182,12 @@ def check(cond: bool, msg: str) -> None:
 
 def check_input(t: torch.Tensor, name: str, dtype: torch.dtype = torch.float32) -> None:
     """CHECK_INPUT of the reference bindings: CUDA, contiguous, dtype."""
-    check(isinstance(t, torch.Tensor) and t.is_cuda, f"{name} must be CUDA")
-    check(t.is_contiguous(), f"{name} must be contiguous")
-    check(t.dtype == dtype, f"{name} must be {str(dtype).replace('torch.', '')}")
+    if not (isinstance(t, torch.Tensor) and t.is_cuda):
+        raise RuntimeError(f"{name} must be CUDA")
+    if not t.is_contiguous():
+        raise RuntimeError(f"{name} must be contiguous")
+    if t.dtype != dtype:
+        raise RuntimeError(f"{name} must be {str(dtype).replace('torch.', '')}")
 
 
 def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
@@ -169,7 +196,10 @@ def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
 
 
 def stream_ptr(device: torch.device | None = None) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    if device is None or device.type != "cuda" or device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    # the handle alone: torch.cuda.current_stream builds a Stream object (3 us)
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 DTYPE_CODE = {torch.float32: 0, torch.bfloat16: 1}

@@ -33,9 +33,12 @@ def _check(cond: bool, msg: str) -> None:
 
 
 def _check_dev(t: torch.Tensor, name: str, dtypes) -> None:
-    _check(t.is_cuda, f"{name} must be CUDA")
-    _check(t.is_contiguous(), f"{name} must be contiguous")
-    _check(t.dtype in dtypes, f"{name} must be {' or '.join(str(d).replace('torch.', '') for d in dtypes)}")
+    if not t.is_cuda:
+        raise RuntimeError(f"{name} must be CUDA")
+    if not t.is_contiguous():
+        raise RuntimeError(f"{name} must be contiguous")
+    if t.dtype not in dtypes:
+        raise RuntimeError(f"{name} must be {' or '.join(str(d).replace('torch.', '') for d in dtypes)}")
 
 
 _F32 = (torch.float32,)

@@ -9,6 +9,7 @@ and cached per row-pointer tensor for the stateless GAT entry points.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import weakref
 from dataclasses import dataclass
 
@@ -66,9 +67,12 @@ class RowSchedule:
     n_hrow: int
     max_degree: int
 
+    def __post_init__(self):
+        self.header_ptr = self.header.ctypes.data  # of the array held here
+
     def args(self):
         """(device schedule, host header) pointers of the C-ABI."""
-        return (self.buf.data_ptr(), self.header.ctypes.data)
+        return (self.buf.data_ptr(), self.header_ptr)
 
 
 def build_row_schedule(rowptr: torch.Tensor, device=None, light_max: int = LIGHT_MAX,
@@ -124,10 +128,17 @@ def gat_schedule(rowptr: torch.Tensor, pass_: int, dtype_code: int, heads: int, 
     the library accepts any multiple of 256 as the segment length (its
     feature-layout kernels, seg_edges reported as 0 = "any"), the length
     follows the graph size like the SpMM's (from SEG_EDGES)."""
+    light, seg = _gat_params(int(pass_), int(dtype_code), int(heads), int(channels))
+    if seg > 0:
+        return cached_row_schedule(rowptr, light, seg)
+    return cached_row_schedule(rowptr, light, None, SEG_EDGES)
+
+
+@functools.lru_cache(maxsize=4096)
+def _gat_params(pass_: int, dtype_code: int, heads: int, channels: int) -> tuple[int, int]:
+    """(light_max, seg_edges) of cign_gat_schedule_params, a function of its
+    arguments alone."""
     lib = load_library(require_gpu=False)
     light, seg = C.c_int32(), C.c_int32()
-    lib.call("cign_gat_schedule_params", int(pass_), int(dtype_code), int(heads), int(channels), C.byref(light),
-             C.byref(seg))
-    if seg.value > 0:
-        return cached_row_schedule(rowptr, light.value, seg.value)
-    return cached_row_schedule(rowptr, light.value, None, SEG_EDGES)
+    lib.call("cign_gat_schedule_params", pass_, dtype_code, heads, channels, C.byref(light), C.byref(seg))
+    return light.value, seg.value

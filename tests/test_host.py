@@ -305,3 +305,29 @@ def test_ctypes_signatures_match_header():
             assert sig_ret in (C.c_void_p, C.c_char_p), name
         else:
             assert C.sizeof(kind(ret)) == C.sizeof(sig_ret), f"{name}: returns {ret}, ctypes {sig_ret}"
+
+
+def test_native_binding_matches_the_library():
+    """_cign.so has every entry point but the two runtime ones, converts as
+    ctypes does (None and addresses, wrapped integers) and turns what it
+    cannot convert, or a wrong argument count, into TypeError."""
+    lib = _lib.load_library(require_gpu=False)
+    from cign_amd import _cign
+
+    entries = {n for n in dir(_cign) if n.startswith("cign_")}
+    assert entries == set(_lib._SIGNATURES) - {"cign_last_error", "cign_version"}
+    for args in ((5, 64), (0, 1), (1 << 20, 4096)):
+        assert _cign.cign_spmm_partial_bytes(*args) == lib._h.cign_spmm_partial_bytes(*args)
+    rowptr = np.array([0, 3, 3, 80], dtype=np.int64)
+    s = build_row_schedule(torch.from_numpy(rowptr), device="cpu")
+    out = np.zeros(s.buf.numel(), dtype=np.int32)
+    args = (rowptr.ctypes.data, 3, LIGHT_MAX, SEG_EDGES, out.ctypes.data)
+    assert _cign.cign_row_schedule_build(*args, out.size) == 0 and np.array_equal(out, s.buf.numpy())
+    assert _cign.cign_row_schedule_build(*args[:-1], None, out.size) == 1  # a null pointer is refused, not read
+    with pytest.raises(RuntimeError, match="buffer size mismatch"):
+        lib.call("cign_row_schedule_build", *args, out.size - 1)
+    for bad in ((5,), (5, 64, 1), ("5", 64)):
+        with pytest.raises(TypeError):
+            _cign.cign_spmm_partial_bytes(*bad)
+    with pytest.raises(TypeError, match="address"):
+        _cign.cign_row_schedule_build("x", 3, LIGHT_MAX, SEG_EDGES, out.ctypes.data, out.size)
