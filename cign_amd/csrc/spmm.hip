@@ -15,9 +15,10 @@
 // their XCDs (workgroup ids go round-robin to the 8 XCDs), so that an XCD's
 // 4 MB L2 holds more of the rows' slices it gathers (launch_all). 24,492
 // nodes, 220,420 entries, fp32, us per hop forward / backward, untiled ->
-// tiled: D = 512 56.1 / 61.9 -> 48.0 / 54.5 (8 tiles of 256 bytes), 384 40.5 /
-// 44.0 -> 36.5 / 39.8, 256 26.6 / 28.7 -> 24.6 / 26.6, 192 21.2 / 22.6 ->
-// 19.4 / 20.9; 2,000 nodes, D = 512: 14.4 -> 8.5 (too few wavefronts untiled).
+// tiled: D = 512 56.1 / 61.9 -> 45.8 / 52.3 (8 tiles of 256 bytes), 384 40.5 /
+// 44.0 -> 35.0 / 38.4, 256 26.6 / 28.7 -> 23.8 / 26.2; 2,000 nodes, D = 512:
+// 14.4 -> 10.2 (too few wavefronts untiled); 60,000 nodes of 26 entries, D =
+// 512: 394 / 407 -> 340 / 365.
 //
 // A row's output is owned by a group of L lanes (L = power of two covering
 // the tile's chunks, 16-byte loads, lane l owns chunks l, l + L, ...). Three
@@ -297,17 +298,33 @@ __global__ __launch_bounds__(kSpmmBlock) void spmm_kernel(SpmmArgs<T, W, VPL, TI
       if (lane < a.L) write_row(a, r.x, gl, acc, ar);
       return;
     }
-    // Tiny rows (degree <= L): one per lane group.
+    // Tiny rows (degree <= L; in tiled launches every light row): one per lane
+    // group.
     const int li = a.n_mid + ((b - a.mid_blocks) * kSpmmWaves + wave) * G + g;
     const bool has = li < s.n_light;
     const int4 r = has ? s.light[li] : make_int4(0, 0, 0, 0);
     const int deg = r.z - r.y;
     const bool mine = gl < deg;
-    const int jj = mine ? a.col[r.y + gl] : 0;
-    const float vv = mine ? a.val[r.y + gl] : 0.0f;
+    int jj = mine ? a.col[r.y + gl] : 0;
+    float vv = mine ? a.val[r.y + gl] : 0.0f;
     AddRow<T, W, VPL, TILED> ar;
     ar.load(a, r.x, gl);  // (row 0 for a group with no row: read, unused)
-    gather(a, jj, vv, g << a.lgL, 0, 1, deg, wave_max_over_groups(deg, a.L), gl, acc);
+    if constexpr (TILED) {
+      // Every light row, L edges a round (the next round's indices loaded
+      // ahead); the wavefront's rows have about the same degree. A row's terms
+      // are then added in edge order, as in a launch of one tile.
+      const int top = wave_max_over_groups(deg, a.L);
+      for (int k = 0; k < top; k += a.L) {
+        const int kn = k + a.L + gl;
+        const int jn = kn < deg ? a.col[r.y + kn] : jj;
+        const float vn = kn < deg ? a.val[r.y + kn] : 0.0f;
+        gather(a, jj, vv, g << a.lgL, 0, 1, max(0, min(deg - k, a.L)), min(top - k, a.L), gl, acc);
+        jj = jn;
+        vv = vn;
+      }
+    } else {
+      gather(a, jj, vv, g << a.lgL, 0, 1, deg, wave_max_over_groups(deg, a.L), gl, acc);
+    }
     // A group's slots past its row's end reload an edge of that row; a row with
     // no edge has read another row's.
     if (deg == 0) zero(acc);
@@ -421,7 +438,7 @@ int launch_tiles(hipStream_t stream, const Sched& s, const SchedInfo& info, int 
   const int G = kWave / a.L;
   // Rows with degree <= L go one per lane group (tiny); the rest of the
   // light list (sorted by degree, descending) one per wavefront.
-  const int n_mid = (G > 1 && a.L >= 8) ? sched_count_gt(info.hdr, a.L) : info.n_light;
+  const int n_mid = TILED ? 0 : (G > 1 && a.L >= 8) ? sched_count_gt(info.hdr, a.L) : info.n_light;
   a.n_mid = n_mid;
   a.mid_blocks = (n_mid + kSpmmWaves - 1) / kSpmmWaves;
   const int n_tiny = info.n_light - n_mid;
@@ -439,18 +456,18 @@ int launch_all(hipStream_t stream, const Sched& s, const SchedInfo& info, int ld
   const int total_ch = (ld + W - 1) / W;
   constexpr int kMaxCh = kWave * 4;  // chunks per launch
   constexpr int kChunkBytes = static_cast<int>(sizeof(T)) * W;
-  constexpr bool kTiles = W > 1 && (std::is_same<T, float>::value || std::is_same<T, bf16>::value);
-  constexpr int kTileBytes = sizeof(T) == 4 ? 256 : 512;
+  constexpr bool kTiles = W > 1 && std::is_same<T, float>::value;
+  constexpr int kTileBytes = 256;
   for (int ch0 = 0; ch0 < total_ch; ch0 += kMaxCh) {
     const int nch = min(kMaxCh, total_ch - ch0);
     const int c0 = ch0 * W;
-    // Column tiles of one launch: up to 8, none narrower than kTileBytes (a
-    // bf16 lane unpacks twice the values of a load, so its narrow tiles cost
-    // more issue than they save latency: D = 512 29.4 us untiled, 27.3 in two
-    // tiles of 512 bytes, 29.2 in four). Rows of at most 512 bytes stay whole
-    // (fp32 D = 128: 13.5 us either way), and so do rows that are no whole
-    // number of 128-byte lines, whose tiles would share lines (fp32 D = 200:
-    // 22.8 us whole, 24.0 in two tiles).
+    // Column tiles of one launch: up to 8, none narrower than 256 bytes (two
+    // tiles of 128 at D = 64: 10.9 us against 8.8). Rows of at most 512 bytes
+    // stay whole (D = 128: 13.5 us either way), and so do rows that are no
+    // whole number of 128-byte lines, whose tiles would share lines (D = 200:
+    // 22.8 us whole, 24.0 in two tiles), and bf16 rows, whose lanes unpack
+    // twice the values of a load (D = 512: 29.4 us whole or in two tiles, 46.8
+    // in eight).
     int lgT = 0;
     if constexpr (kTiles) {
       if (nch * kChunkBytes > 512 && (ld * static_cast<int>(sizeof(T))) % 128 == 0)

@@ -269,8 +269,8 @@ def test_spmm_big_hubs_segment_sizes(seg_edges, dtype, d):
     assert int(parts.sched.counters.abs().sum()) == 0
 
 
-# Widths at the edges of the column tiling (rows of 512 bytes and less whole,
-# then 2, 4 and 8 tiles, more than one launch) and rows without 16-byte
+# Widths at the edges of the fp32 column tiling (rows of 512 bytes and less
+# whole, then 2, 4 and 8 tiles, more than one launch) and rows without 16-byte
 # alignment (the last chunk overlaps the one before it).
 @pytest.mark.parametrize("dtype,d", [(torch.float32, d) for d in
                                      (4, 5, 33, 63, 128, 129, 160, 192, 333, 384, 512, 544, 1023, 1027, 2048)] +
