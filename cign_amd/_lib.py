@@ -51,6 +51,9 @@ _SIGNATURES = {
                                      _U64, _P, _P, _P, _P, _P, _P, _I64, _P, _I64, _I64]),
     "cign_gat_bwd_shard": (C.c_int, [_P, _I32, _I32, _I32, _I32, _I32, _F32, _F32] + [_P] * 11
                            + [_P, _P, _P, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _I32, _I32, _I64]),
+    "cign_gat_bwd_logits_ok": (C.c_int, [_I32, _I32, _I32, _I64]),
+    "cign_gat_bwd_logits": (C.c_int, [_P, _I32, _I32, _I32, _I32, _I32, _F32, _F32] + [_P] * 11
+                            + [_P, _P, _P, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _P, _P]),
     # GAT side ops and block ops (nodeops.hip)
     "cign_colsum_workspace_bytes": (_I64, [_I64, _I32, _I32]),
     "cign_attn_logits_fwd": (C.c_int, [_P, _I64, _I32, _I32, _P, _P, _P, _P, _P]),
@@ -58,6 +61,7 @@ _SIGNATURES = {
     "cign_attn_logits_fwd_bf16": (C.c_int, [_P, _I64, _I32, _I32, _P, _P, _P, _P, _P]),
     "cign_attn_logits_bwd_acc": (C.c_int, [_P, _I64, _I32, _I32, _I32, _I32, _P, _P, _P, _P, _P, _P, _P, _P, _P,
                                            _P, _I64]),
+    "cign_attn_vec_grad": (C.c_int, [_P, _I64, _I32, _I32, _I32] + [_P] * 8 + [_I64]),
     "cign_head_silu_fwd": (C.c_int, [_P, _I64, _I32, _I32, _P, _P, _P, _P]),
     "cign_head_silu_bwd": (C.c_int, [_P, _I64, _I32, _I32, _P, _P, _P, _P, _P, _I64]),
     "cign_dropout_ln_fwd": (C.c_int, [_P, _I64, _I32, _P, _P, _P, _F32, _F32, _U64, _P, _P, _P, _P]),
@@ -118,7 +122,7 @@ class _Lib:
             fn.restype = res
             fn.argtypes = args
             self._fn[name] = fn if name in _BY_REFERENCE else getattr(native, name, fn)
-            sizes = name.endswith(("_bytes", "_floats"))
+            sizes = name.endswith(("_bytes", "_floats", "_ok"))
             setattr(self, name, self._fn[name] if sizes else fn)
 
     def call(self, name: str, *args) -> None:

@@ -121,10 +121,14 @@ class _CollapsedGATExt:
 
     @staticmethod
     def backward(negative_slope, attn_drop, row_ptr, col_ind, col_ptr, row_ind, permute, edge_max, edge_sum,
-                 edge_mask, in_feat, attn_row, attn_col, pre, grad_y, row_agg=None, f32_out=False):
+                 edge_mask, in_feat, attn_row, attn_col, pre, grad_y, row_agg=None, f32_out=False, logits=None):
         """``row_agg``: the buffer forward_agg() returned for the same inputs,
         or None (the rows pass then gathers in_feat per edge). ``f32_out``
-        as in forward_agg: grad_y and grad_feat are float32."""
+        as in forward_agg: grad_y and grad_feat are float32. ``logits`` =
+        (att_src, att_dst), float32 [H*C] values, where
+        cign_gat_bwd_logits_ok: the first result is then the gradient of the
+        projection in_feat is, the logits' gradients of it included
+        (float32, or bfloat16 with ``f32_out``)."""
         for t, n in ((row_ptr, "row_ptr"), (col_ind, "col_ind"), (col_ptr, "col_ptr"), (row_ind, "row_ind"),
                      (permute, "permute")):
             _check_dev(t, n, _I32)
@@ -147,16 +151,19 @@ class _CollapsedGATExt:
         row_blocks = rs.n_seg + (rs.n_light + 3) // 4
         ws_bytes = int(lib.cign_gat_bwd_workspace_bytes(n, nnz, H, C, row_blocks, rs.n_seg, cs.n_seg))
         ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-        grad_feat = torch.empty_like(in_feat, dtype=torch.float32 if code == 2 else in_feat.dtype)
+        gf_dtype = torch.float32 if code == 2 and logits is None else in_feat.dtype
+        grad_feat = torch.empty_like(in_feat, dtype=gf_dtype)
         grad_attn_row = torch.empty_like(attn_row)
         grad_attn_col = torch.empty_like(attn_col)
         grad_bias = torch.empty((C,), dtype=torch.float32, device=dev)
-        lib.call("cign_gat_bwd", _lib.stream_ptr(dev), code, n, nnz, H, C, float(negative_slope),
+        entry = "cign_gat_bwd" if logits is None else "cign_gat_bwd_logits"
+        vectors = () if logits is None else (logits[0].data_ptr(), logits[1].data_ptr())
+        lib.call(entry, _lib.stream_ptr(dev), code, n, nnz, H, C, float(negative_slope),
                  float(attn_drop), col_ind.data_ptr(), row_ind.data_ptr(),
                  permute.data_ptr(), edge_max.data_ptr(), edge_sum.data_ptr(), edge_mask.data_ptr(),
                  in_feat.data_ptr(), attn_row.data_ptr(), attn_col.data_ptr(), pre.data_ptr(), grad_y.data_ptr(),
                  *rs.args(), rs.counters.data_ptr(), *cs.args(), cs.counters.data_ptr(), ws.data_ptr(), ws_bytes,
-                 grad_feat.data_ptr(), grad_attn_row.data_ptr(), grad_attn_col.data_ptr(), grad_bias.data_ptr(),
+                 *vectors, grad_feat.data_ptr(), grad_attn_row.data_ptr(), grad_attn_col.data_ptr(), grad_bias.data_ptr(),
                  _lib.ptr(row_agg))
         return [grad_feat, grad_attn_row, grad_attn_col, grad_bias]
 

@@ -367,7 +367,8 @@ int gat_bwd_impl(void* stream, int32_t dtype, int32_t n, int32_t nnz, int32_t he
                  int32_t* row_counters, const int32_t* col_sched, const int32_t* col_sched_info,
                  int32_t* col_counters, void* workspace, int64_t workspace_bytes, void* grad_feat,
                  float* grad_attn_row, float* grad_attn_col, float* grad_bias, const float* row_agg,
-                 int32_t bias_lo, int32_t bias_n, int64_t graph_nnz) {
+                 int32_t bias_lo, int32_t bias_n, int64_t graph_nnz, const float* att_src = nullptr,
+                 const float* att_dst = nullptr) {
   int rc = check_shape("cign_gat_bwd", n, nnz, heads, channels);
   if (row_agg && (cign_gat_row_agg_floats(dtype, n, heads, channels) == 0 || !aligned16(row_agg)))
     return set_error(kInvalid, "cign_gat_bwd: row_agg must be null for this shape (cign_gat_row_agg_floats) or "
@@ -413,6 +414,7 @@ int gat_bwd_impl(void* stream, int32_t dtype, int32_t n, int32_t nnz, int32_t he
     a.part_row = reinterpret_cast<float*>(ws + L.part_row);
     a.part_col = reinterpret_cast<float*>(ws + L.part_col);
     a.row_counters = row_counters; a.col_counters = col_counters;
+    a.att_src = att_src; a.att_dst = att_dst;
     a.grad_feat = gxt; a.grad_attn_row = grad_attn_row; a.grad_attn_col = grad_attn_col; a.grad_bias = grad_bias;
     int FL, FV;
     bool exact;
@@ -495,6 +497,32 @@ int cign_gat_bwd_shard(void* stream, int32_t dtype, int32_t n, int32_t nnz, int3
                       edge_sum, edge_mask, in_feat, attn_row, attn_col, pre, grad_y, row_sched, row_sched_info,
                       row_counters, col_sched, col_sched_info, col_counters, workspace, workspace_bytes, grad_feat,
                       grad_attn_row, grad_attn_col, grad_bias, row_agg, bias_row_lo, bias_rows, graph_nnz);
+}
+
+// Whether cign_gat_bwd_logits takes this shape and graph.
+int cign_gat_bwd_logits_ok(int32_t dtype, int32_t heads, int32_t channels, int64_t nnz) {
+  if ((dtype != kF32 && dtype != kBF16F32) || !fl_ok(dtype, heads, channels)) return 0;
+  // the channel-major columns kernel writes grad_feat alone
+  return !(cols_cm_ok(heads, channels) && nnz >= big_graph_edges());
+}
+
+int cign_gat_bwd_logits(void* stream, int32_t dtype, int32_t n, int32_t nnz, int32_t heads, int32_t channels,
+                        float negative_slope, float attn_drop, const int32_t* col, const int32_t* rowind,
+                        const int32_t* perm, const float* edge_max, const float* edge_sum, const uint8_t* edge_mask,
+                        const void* in_feat, const float* attn_row, const float* attn_col, const float* pre,
+                        const void* grad_y, const int32_t* row_sched, const int32_t* row_sched_info,
+                        int32_t* row_counters, const int32_t* col_sched, const int32_t* col_sched_info,
+                        int32_t* col_counters, void* workspace, int64_t workspace_bytes, const float* att_src,
+                        const float* att_dst, void* grad_proj, float* grad_attn_row, float* grad_attn_col,
+                        float* grad_bias, const float* row_agg) {
+  if (!cign_gat_bwd_logits_ok(dtype, heads, channels, nnz))
+    return set_error(kInvalid, "cign_gat_bwd_logits: dtype %d, heads=%d channels=%d, %d edges not taken "
+                     "(cign_gat_bwd_logits_ok)", dtype, heads, channels, nnz);
+  if (!att_src || !att_dst) return set_error(kInvalid, "cign_gat_bwd_logits: null att_src / att_dst");
+  return gat_bwd_impl(stream, dtype, n, nnz, heads, channels, negative_slope, attn_drop, col, rowind, perm, edge_max,
+                      edge_sum, edge_mask, in_feat, attn_row, attn_col, pre, grad_y, row_sched, row_sched_info,
+                      row_counters, col_sched, col_sched_info, col_counters, workspace, workspace_bytes, grad_proj,
+                      grad_attn_row, grad_attn_col, grad_bias, row_agg, 0, n, nnz, att_src, att_dst);
 }
 
 }  // extern "C"

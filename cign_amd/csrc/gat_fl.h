@@ -1444,6 +1444,28 @@ __device__ __forceinline__ void load_attn_col(const GatBwdArgs<T>& a, const FlLa
   }
 }
 
+// The logits' gradients in the columns' stores (GatBwdArgs::att_src): the
+// column's grad_attn_col is at hand and its grad_attn_row is the rows pass's,
+// so the sum costs two 16-byte loads a chunk (the vectors, cached) where a pass
+// of its own read grad_feat, 150 MB of fp32 at 24,492 x 6 x 256, and wrote the
+// sum. bf16 features: columns 75 + logits' backward 52 us -> 73 + 19 (the
+// vectors' gradients alone), and grad_proj in 2 bytes; fp32 87 + 74 -> 94 + 31.
+// Type of the projection's gradient: bf16 for bf16x.
+template <typename T>
+using GatProj = std::conditional_t<std::is_same_v<T, bf16x>, bf16, GatOut<T>>;
+// Whether T's launches may carry att_src / att_dst.
+template <typename T>
+constexpr bool kGatProj = std::is_same_v<T, float> || std::is_same_v<T, bf16x>;
+
+// Element k = h C + c of column j's projection gradient from its grad_feat
+// value v and the column's grad_attn_col of head h.
+template <typename T>
+__device__ __forceinline__ void store_proj1(const GatBwdArgs<T>& a, int j, int h, int k, float v, float gac) {
+  const float gar = a.grad_attn_row[static_cast<int64_t>(j) * a.H + h];
+  const float g = v + (gac * a.att_src[k] + gar * a.att_dst[k]);
+  reinterpret_cast<GatProj<T>*>(a.grad_feat)[static_cast<int64_t>(j) * a.H * a.C + k] = from_f32<GatProj<T>>(g);
+}
+
 template <typename T, int L, int V, bool DROP, int R>
 __global__ __launch_bounds__(kBlock) void gat_bwd_cols_fl_kernel(GatBwdArgs<T> a, Sched s, int n_mid, int mid_blocks,
                                                                  int lgcq) {
@@ -1509,7 +1531,21 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_cols_fl_kernel(GatBwdArgs<T> a
       float o[W];
 #pragma unroll
       for (int w = 0; w < W; ++w) o[w] = st.ug[v][w] * a.inv_h;
-      store_values<GatOut<T>, W>(a.grad_feat + static_cast<int64_t>(j) * F + ln.off[v], o);
+      bool plain = true;
+      if constexpr (kGatProj<T>) {
+        if (a.att_src) {  // uniform
+          plain = false;
+          const float gar = a.grad_attn_row[static_cast<int64_t>(j) * a.H + ln.hq[v]];
+          float as[W], ad[W];
+          load_f32<W>(a.att_src + ln.off[v], as);
+          load_f32<W>(a.att_dst + ln.off[v], ad);
+#pragma unroll
+          for (int w = 0; w < W; ++w) o[w] += gac[v] * as[w] + gar * ad[w];
+          store_values<GatProj<T>, W>(
+              reinterpret_cast<GatProj<T>*>(a.grad_feat) + static_cast<int64_t>(j) * F + ln.off[v], o);
+        }
+      }
+      if (plain) store_values<GatOut<T>, W>(a.grad_feat + static_cast<int64_t>(j) * F + ln.off[v], o);
       if (ln.cw == 0) a.grad_attn_col[static_cast<int64_t>(j) * a.H + ln.hq[v]] = gac[v];
     }
     return;
@@ -1559,11 +1595,22 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_cols_fl_kernel(GatBwdArgs<T> a
   }
   const bool single = hr.y == 1;
   const int stride = F + a.H;
+  bool proj = false;
+  if constexpr (kGatProj<T>) proj = a.att_src != nullptr;
+  // (the loops above end in a barrier: red and gred are complete)
   float* mine = a.part_col + static_cast<int64_t>(b) * stride;
   for (int k = threadIdx.x; k < F; k += kBlock) {
     const float v = red[k];
-    if (single) a.grad_feat[static_cast<int64_t>(j) * F + k] = from_f32<GatOut<T>>(v * a.inv_h);
-    else st_agent(mine + k, v);
+    if (!single) {
+      st_agent(mine + k, v);
+    } else if (proj) {
+      if constexpr (kGatProj<T>) {
+        const int h = k / a.C;
+        store_proj1(a, j, h, k, v * a.inv_h, gred[0][h] + gred[1][h] + gred[2][h] + gred[3][h]);
+      }
+    } else {
+      a.grad_feat[static_cast<int64_t>(j) * F + k] = from_f32<GatOut<T>>(v * a.inv_h);
+    }
   }
   if (threadIdx.x < a.H) {
     const int h = threadIdx.x;
@@ -1573,11 +1620,21 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_cols_fl_kernel(GatBwdArgs<T> a
   }
   if (single) return;
   if (!arrive_last(a.col_counters + sg.w, hr.y, &flag)) return;
-  for (int k = threadIdx.x; k < stride; k += kBlock) {
+  if (threadIdx.x < a.H) {
+    float v = 0.0f;
+    for (int z = 0; z < hr.y; ++z) v += ld_agent(a.part_col + static_cast<int64_t>(hr.x + z) * stride + F + threadIdx.x);
+    a.grad_attn_col[static_cast<int64_t>(j) * a.H + threadIdx.x] = v;
+    gred[0][threadIdx.x] = v;
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k < F; k += kBlock) {
     float v = 0.0f;
     for (int z = 0; z < hr.y; ++z) v += ld_agent(a.part_col + static_cast<int64_t>(hr.x + z) * stride + k);
-    if (k < F) a.grad_feat[static_cast<int64_t>(j) * F + k] = from_f32<GatOut<T>>(v * a.inv_h);
-    else a.grad_attn_col[static_cast<int64_t>(j) * a.H + (k - F)] = v;
+    if (proj) {
+      if constexpr (kGatProj<T>) store_proj1(a, j, k / a.C, k, v * a.inv_h, gred[0][k / a.C]);
+    } else {
+      a.grad_feat[static_cast<int64_t>(j) * F + k] = from_f32<GatOut<T>>(v * a.inv_h);
+    }
   }
 }
 

@@ -498,6 +498,12 @@ struct GatBwdArgs {
   int32_t* col_counters;  // [n_hrow_cols + 1]; last slot = bias counter
   int rows_blocks;
   int n_l2;
+  // Optional (feature layout, head-major columns, T float or bf16x): the
+  // logits' vectors [H, C]. grad_feat then receives the whole gradient of the
+  // projection, grad_feat + grad_attn_col att_src + grad_attn_row att_dst, in
+  // float for T = float, rounded to bf16 for bf16x.
+  const float* att_src;
+  const float* att_dst;
   // outputs
   GatOut<T>* grad_feat;
   float* grad_attn_row;

@@ -299,7 +299,7 @@ __global__ __launch_bounds__(kBlock) void attn_fwd_kernel(int64_t rows, int H, i
 
 // Rows = nodes of width F = H*C; column tile blockIdx.y of LPR*V chunks.
 // Writes g_x (plus gx_in, the gradient x receives from its other consumer,
-// when not null; it may alias gx) and the tile's partial sums of gs*x and
+// when not null; it may alias gx) unless gx is null, and the tile's partial sums of gs*x and
 // gd*x for row block blockIdx.x (part layout [2][nb][F]).
 template <int LPR, int V, int W, typename TX = float, typename TO = float>
 __global__ __launch_bounds__(kBlock) void attn_bwd_kernel(int64_t n, int H, int C, const float* gs, const float* gd,
@@ -342,7 +342,7 @@ __global__ __launch_bounds__(kBlock) void attn_bwd_kernel(int64_t n, int H, int 
           accs[v][w] = fmaf(s, xv[w], accs[v][w]);
           accd[v][w] = fmaf(d, xv[w], accd[v][w]);
         }
-        Chunk<TO, W>::store(gx + r * F + c * W, o);
+        if (gx) Chunk<TO, W>::store(gx + r * F + c * W, o);
       }
     }
   }
@@ -893,6 +893,19 @@ int cign_attn_logits_bwd_acc(void* stream, int64_t n, int32_t H, int32_t C, int3
     return attn_bwd_impl(who, stream, n, H, C, grad_src, grad_dst, static_cast<const bf16h*>(x), att_src, att_dst,
                          grad_x_in, gx, grad_att_src, grad_att_dst, workspace, workspace_bytes,
                          grad_x_dtype == kBF16);
+  return set_error(kInvalid, "%s: x_dtype must be 0 (float32) or 1 (bf16), got %d", who, x_dtype);
+}
+
+int cign_attn_vec_grad(void* stream, int64_t n, int32_t H, int32_t C, int32_t x_dtype, const float* grad_src,
+                       const float* grad_dst, const void* x, const float* att_src, const float* att_dst,
+                       float* grad_att_src, float* grad_att_dst, void* workspace, int64_t workspace_bytes) {
+  const char* who = "cign_attn_vec_grad";
+  if (x_dtype == kF32)
+    return attn_bwd_impl(who, stream, n, H, C, grad_src, grad_dst, static_cast<const float*>(x), att_src, att_dst,
+                         nullptr, nullptr, grad_att_src, grad_att_dst, workspace, workspace_bytes);
+  if (x_dtype == kBF16)
+    return attn_bwd_impl(who, stream, n, H, C, grad_src, grad_dst, static_cast<const bf16h*>(x), att_src, att_dst,
+                         nullptr, nullptr, grad_att_src, grad_att_dst, workspace, workspace_bytes);
   return set_error(kInvalid, "%s: x_dtype must be 0 (float32) or 1 (bf16), got %d", who, x_dtype);
 }
 

@@ -76,11 +76,14 @@ PyMethodDef methods[] = {
     CIGN_ENTRY(cign_gat_bwd),
     CIGN_ENTRY(cign_gat_fwd_shard),
     CIGN_ENTRY(cign_gat_bwd_shard),
+    CIGN_ENTRY(cign_gat_bwd_logits_ok),
+    CIGN_ENTRY(cign_gat_bwd_logits),
     CIGN_ENTRY(cign_colsum_workspace_bytes),
     CIGN_ENTRY(cign_attn_logits_fwd),
     CIGN_ENTRY(cign_attn_logits_bwd),
     CIGN_ENTRY(cign_attn_logits_fwd_bf16),
     CIGN_ENTRY(cign_attn_logits_bwd_acc),
+    CIGN_ENTRY(cign_attn_vec_grad),
     CIGN_ENTRY(cign_head_silu_fwd),
     CIGN_ENTRY(cign_head_silu_bwd),
     CIGN_ENTRY(cign_dropout_ln_fwd),

@@ -123,17 +123,29 @@ class _LinGatFn(torch.autograd.Function):
         ext = ensure_collapsed_gat_loaded(False)
         M, H, C = xp.shape
         dev = xp.device
+        K = x2.size(1)
+        fused_wgrad = (not ctx.needs_input_grad[0] and _SMALL_N < H * C <= _NARROW_N and C % 4 == 0 and K % 4 == 0
+                       and x2.dtype == torch.float32 and x2.is_contiguous() and x2.data_ptr() % 16 == 0)
+        # With x_proj held in bf16 the summed gradient of x_proj is written
+        # rounded to bf16, the values the projection's bf16-math backward
+        # reads of it.
+        gy16 = ctx.hold and C % 8 == 0 and H * C > _SMALL_N
+        # The GAT's columns pass adds the logits' gradients as it writes its
+        # own, where it can; otherwise the logits' backward reads it back
+        # (columns + logits' backward at 24,492 nodes x 6 x 256: bf16 127 us,
+        # 92 with the sum in the columns; fp32 162, 125).
+        in_columns = (not fused_wgrad and gy16 == ctx.hold
+                      and lib.cign_gat_bwd_logits_ok(2 if ctx.hold else 0, H, C, col.numel()))
         grad_feat, g_attn_row, g_attn_col, g_bias = ext.backward(
             ctx.negative_slope, ctx.attn_drop, rowptr, col, colptr, row, perm, edge_max, edge_sum, edge_mask, xp,
-            a_dst, a_src, pre, grad_y.float().contiguous(), agg, f32_out=ctx.hold)
+            a_dst, a_src, pre, grad_y.float().contiguous(), agg, f32_out=ctx.hold,
+            logits=(s, d) if in_columns else None)
         # d alpha_src is the GAT's attn_col gradient, d alpha_dst its attn_row
         # gradient; the logits' term is added to grad_feat in place.
         g_s = torch.empty_like(s)
         g_d = torch.empty_like(d)
         st = _lib.stream_ptr(dev)
-        K = x2.size(1)
-        if (not ctx.needs_input_grad[0] and _SMALL_N < H * C <= _NARROW_N and C % 4 == 0 and K % 4 == 0
-                and x2.dtype == torch.float32 and x2.is_contiguous() and x2.data_ptr() % 16 == 0):
+        if fused_wgrad:
             # input features that are data (config c2): the logits' backward
             # fused into the weight gradient, gy never stored
             gw = torch.empty((H * C, K), dtype=torch.float32, device=dev)
@@ -143,17 +155,19 @@ class _LinGatFn(torch.autograd.Function):
                      g_attn_col.data_ptr(), g_attn_row.data_ptr(), xp.data_ptr(), s.data_ptr(), d.data_ptr(),
                      x2.data_ptr(), gw.data_ptr(), g_s.data_ptr(), g_d.data_ptr(), ws.data_ptr(), ws_bytes)
             return (None, gw if ctx.needs_input_grad[1] else None, g_s, g_d, g_bias) + (None,) * 10
-        # With x_proj held in bf16 the sum is written rounded to bf16, the
-        # values the projection's bf16-math backward reads of it.
-        gy16 = ctx.hold and C % 8 == 0 and H * C > _SMALL_N
-        gy = torch.empty((M, H, C), dtype=torch.bfloat16, device=dev) if gy16 else grad_feat
         ws_bytes = int(lib.cign_colsum_workspace_bytes(M, H * C, 2))
         ws = _lib.workspace(ws_bytes, dev)
-        lib.call("cign_attn_logits_bwd_acc", st, M, H, C, 1 if ctx.hold else 0, 1 if gy16 else 0,
-                 g_attn_col.data_ptr(), g_attn_row.data_ptr(), xp.data_ptr(), s.data_ptr(), d.data_ptr(),
-                 grad_feat.data_ptr(), gy.data_ptr(), g_s.data_ptr(), g_d.data_ptr(), ws.data_ptr(), ws_bytes)
+        if in_columns:
+            gy = grad_feat
+            lib.call("cign_attn_vec_grad", st, M, H, C, 1 if ctx.hold else 0, g_attn_col.data_ptr(),
+                     g_attn_row.data_ptr(), xp.data_ptr(), s.data_ptr(), d.data_ptr(), g_s.data_ptr(), g_d.data_ptr(),
+                     ws.data_ptr(), ws_bytes)
+        else:
+            gy = torch.empty((M, H, C), dtype=torch.bfloat16, device=dev) if gy16 else grad_feat
+            lib.call("cign_attn_logits_bwd_acc", st, M, H, C, 1 if ctx.hold else 0, 1 if gy16 else 0,
+                     g_attn_col.data_ptr(), g_attn_row.data_ptr(), xp.data_ptr(), s.data_ptr(), d.data_ptr(),
+                     grad_feat.data_ptr(), gy.data_ptr(), g_s.data_ptr(), g_d.data_ptr(), ws.data_ptr(), ws_bytes)
         if gy16:
-            K = x2.size(1)
             xf = x2 if x2.dtype == torch.float32 else x2.float()
             gx = torch.empty((M, K), dtype=torch.float32, device=dev) if ctx.needs_input_grad[0] else None
             gw = torch.empty((H * C, K), dtype=torch.float32, device=dev)

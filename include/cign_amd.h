@@ -159,6 +159,25 @@ int cign_gat_bwd(void* stream, int32_t dtype, int32_t n, int32_t nnz, int32_t he
                  int32_t* col_counters, void* workspace, int64_t workspace_bytes, void* grad_feat,
                  float* grad_attn_row, float* grad_attn_col, float* grad_bias, const float* row_agg);
 
+/* cign_gat_bwd whose columns pass writes the whole gradient of the projection
+ * that in_feat is, grad_proj = grad_feat + grad_attn_col att_src +
+ * grad_attn_row att_dst (att_src / att_dst [H,C] f32: attn_col = <in_feat,
+ * att_src> and attn_row = <in_feat, att_dst> per head), in place of grad_feat:
+ * float32 for dtype 0, rounded to bf16 for dtype 2. The sum the reference's
+ * autograd forms of the GAT's and the logits' gradients of x_proj
+ * (model_cign.py:546-566), without a pass that reads grad_feat back. Shapes
+ * and graphs for which cign_gat_bwd_logits_ok returns 1. */
+int cign_gat_bwd_logits_ok(int32_t dtype, int32_t heads, int32_t channels, int64_t nnz);
+int cign_gat_bwd_logits(void* stream, int32_t dtype, int32_t n, int32_t nnz, int32_t heads, int32_t channels,
+                        float negative_slope, float attn_drop, const int32_t* col, const int32_t* rowind,
+                        const int32_t* perm, const float* edge_max, const float* edge_sum, const uint8_t* edge_mask,
+                        const void* in_feat, const float* attn_row, const float* attn_col, const float* pre,
+                        const void* grad_y, const int32_t* row_sched, const int32_t* row_sched_info,
+                        int32_t* row_counters, const int32_t* col_sched, const int32_t* col_sched_info,
+                        int32_t* col_counters, void* workspace, int64_t workspace_bytes, const float* att_src,
+                        const float* att_dst, void* grad_proj, float* grad_attn_row, float* grad_attn_col,
+                        float* grad_bias, const float* row_agg);
+
 /* cign_gat_fwd over one destination-row shard of a larger graph, the
  * partitioned execution that replaces run_chunked_dgnn_op
  * (chunked_dgnn_gat.py:214-252): n and col are the shard's rows and its
@@ -242,6 +261,15 @@ int cign_attn_logits_bwd_acc(void* stream, int64_t n, int32_t heads, int32_t cha
                              int32_t grad_x_dtype, const float* grad_src, const float* grad_dst, const void* x,
                              const float* att_src, const float* att_dst, const float* grad_x_in, void* grad_x,
                              float* grad_att_src, float* grad_att_dst, void* workspace, int64_t workspace_bytes);
+
+/* The logits' vector gradients alone (grad_att_src = sum_n gs x, grad_att_dst
+ * = sum_n gd x): the part of cign_attn_logits_bwd_acc that is left where
+ * cign_gat_bwd_logits has written the gradient of x. Workspace:
+ * cign_colsum_workspace_bytes(n, heads*channels, 2). */
+int cign_attn_vec_grad(void* stream, int64_t n, int32_t heads, int32_t channels, int32_t x_dtype,
+                       const float* grad_src, const float* grad_dst, const void* x, const float* att_src,
+                       const float* att_dst, float* grad_att_src, float* grad_att_dst, void* workspace,
+                       int64_t workspace_bytes);
 
 /* pre = sum_h out[n,h,:] / H + bias, y = SiLU(pre). Replaces ext
  * head_silu_forward (fused_gat_sideops.cpp:68-76; kernel

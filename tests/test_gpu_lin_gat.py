@@ -330,3 +330,69 @@ def test_lin_gat_data_input_fused_wgrad(n, K, amp):
         a, e = res[True][k], res[False][k]
         extra = bf16_flip_atol(e.cpu().numpy()) if amp and k == "lin.weight" else 0.0
         assert_close(a, e, rtol=1e-4, atol=1e-5 * max(1.0, float(e.abs().max())) + extra, name=k)
+
+
+@pytest.mark.parametrize("H,C,hold,p", [(6, 256, True, 0.2), (6, 256, False, 0.0), (4, 64, True, 0.0),
+                                        (4, 16, False, 0.2), (5, 48, False, 0.2), (7, 256, False, 0.0)])
+def test_gat_backward_with_logits(H, C, hold, p):
+    """cign_gat_bwd_logits against cign_gat_bwd followed by the logits'
+    backward, with columns in one and in several segments: the attention and
+    bias gradients bit for bit, the projection's gradient to the rounding of
+    one float32 sum of three terms (and of the bf16 store, when held), the
+    vectors' gradients alone bit for bit."""
+    from cign_amd import _lib
+    from cign_amd.collapsed_gat import ensure_collapsed_gat_loaded
+
+    print(f"gat bwd logits H={H} C={C} hold={hold} p={p}", flush=True)
+    lib = _lib.load_library()
+    code = 2 if hold else 0
+    rng = np.random.default_rng(H * C + hold)
+    n = 1500
+    ei = _graph(rng, n, {2: 1400, 7: 300})
+    out = np.stack([np.full(1400, 11), rng.permutation(n)[:1400]])  # a source of many segments
+    from oracle import cign_oracle as O
+    r, c, _ = O.coalesce(np.concatenate([ei[0], out[0]]), np.concatenate([ei[1], out[1]]), n)
+    ei = np.stack([r, c])
+    rowptr, col, row, colptr, perm = _dev_graph(ei, n)
+    assert int(colptr.diff().max()) > 1024
+    assert lib.cign_gat_bwd_logits_ok(code, H, C, col.numel()) == 1
+    dt = torch.bfloat16 if hold else torch.float32
+    f = lambda *s: torch.from_numpy(rng.standard_normal(s).astype(np.float32)).cuda()
+    x, ar, ac, b, gy, s, d = f(n, H, C).to(dt), f(n, H), f(n, H), f(C), f(n, C), f(H, C), f(H, C)
+    ext = ensure_collapsed_gat_loaded()
+    (_, pre, emax, esum, mask), agg = ext.forward_agg(ar, ac, rowptr, col, 0.2, x, b, p, 9, True, f32_out=hold)
+    args = (0.2, p, rowptr, col, colptr, row, perm, emax, esum, mask, x, ar, ac, pre, gy, agg)
+    gx, g_row, g_col, g_b = ext.backward(*args, f32_out=hold)
+    proj, p_row, p_col, p_b = ext.backward(*args, f32_out=hold, logits=(s, d))
+    assert proj.dtype == dt
+    for a, e in ((p_row, g_row), (p_col, g_col), (p_b, g_b)):
+        assert torch.equal(a, e)
+    terms = [gx.double(), g_col.double()[:, :, None] * s.double(), g_row.double()[:, :, None] * d.double()]
+    want, size = sum(terms), sum(t.abs() for t in terms)
+    bound = 4 * 2.0 ** -24 * size + (2.0 ** -8 * want.abs() if hold else 0.0)
+    assert bool(((proj.double() - want).abs() <= bound).all())
+    st = _lib.stream_ptr(x.device)
+    ws_bytes = int(lib.cign_colsum_workspace_bytes(n, H * C, 2))
+    ws = _lib.workspace(ws_bytes, x.device)
+    vecs = [torch.empty((2, H, C), device="cuda") for _ in range(2)]
+    gxo = torch.empty((n, H, C), device="cuda")
+    xd = 1 if hold else 0
+    lib.call("cign_attn_logits_bwd_acc", st, n, H, C, xd, 0, g_col.data_ptr(), g_row.data_ptr(), x.data_ptr(),
+             s.data_ptr(), d.data_ptr(), gx.data_ptr(), gxo.data_ptr(), vecs[0][0].data_ptr(), vecs[0][1].data_ptr(),
+             ws.data_ptr(), ws_bytes)
+    lib.call("cign_attn_vec_grad", st, n, H, C, xd, g_col.data_ptr(), g_row.data_ptr(), x.data_ptr(), s.data_ptr(),
+             d.data_ptr(), vecs[1][0].data_ptr(), vecs[1][1].data_ptr(), ws.data_ptr(), ws_bytes)
+    assert torch.equal(vecs[0], vecs[1])
+
+
+def test_gat_backward_with_logits_refuses_other_kernels():
+    from cign_amd import _lib
+
+    lib = _lib.load_library()
+    ok = lib.cign_gat_bwd_logits_ok
+    assert ok(0, 4, 16, 10**5) == 1 and ok(2, 6, 256, 10**5) == 1
+    assert ok(0, 4, 15, 10**5) == 0 and ok(0, 12, 16, 10**5) == 0  # pair layout
+    assert ok(2, 6, 40, 10**5) == 0 and ok(1, 4, 16, 10**5) == 0
+    assert ok(0, 4, 16, 1 << 22) == 0 and ok(0, 6, 16, 1 << 22) == 1  # channel-major columns
+    with pytest.raises(RuntimeError, match="not taken"):
+        lib.call("cign_gat_bwd_logits", None, 0, 10, 10, 4, 15, 0.2, 0.0, *([None] * 18), 0, *([None] * 7))
