@@ -2274,7 +2274,7 @@ struct PackArgs {
   int64_t p_stride;  // row stride of the hops (>= 2D)
   const float* alpha;
   int64_t a_stride;  // row stride of alpha: K, or 0 for one row shared by all nodes
-  const __bf16* w16;  // bf16 math: Wp rounded to bf16 once per call [D, 2KD]
+  const __bf16* w16;  // bf16 math, forward: Wp in pack_w16_kernel's order
 };
 
 // Forward A tile of one K step (hop kk, channels j0 .. j0+15): BM rows x 32
@@ -2323,11 +2323,9 @@ struct PackAStage {
   }
 };
 
-// Forward W tile of the same K step: BN rows (all D outputs) x 32, tile
-// column c < 16 from Wp column kk*2D + j0 + c, c >= 16 from kk*2D + D + j0 +
-// c - 16. fp32 math reads Wp; bf16 math its bf16 copy (half the bytes, no
-// conversion per step), 16-byte chunks either way.
-template <int MATH, int BN>
+// Forward W tile of the same K step (fp32 math): BN rows x 32, tile column c <
+// 16 from Wp column kk*2D + j0 + c, c >= 16 from kk*2D + D + j0 + c - 16.
+template <int BN>
 struct PackBStage {
   static constexpr int CHUNKS = BN * kBK / 4 / kThreads;
   float b[CHUNKS][4];
@@ -2351,66 +2349,31 @@ struct PackBStage {
   }
 };
 
-template <int BN>
-struct PackBStage<kMathBF16, BN> {
-  static constexpr int CHUNKS = BN * kBK / 8 / kThreads;
-  bf16x8 b[CHUNKS];
-
-  __device__ __forceinline__ void load(const GemmArgs& g, const PackArgs& a, int kk, int j0, int D, int n0) {
-#pragma unroll
-    for (int i = 0; i < CHUNKS; ++i) {
-      const int id = threadIdx.x + i * kThreads;
-      const int r = id >> 2, c = id & 3;
-      const int col = kk * 2 * D + (c < 2 ? j0 + 8 * c : D + j0 + 8 * (c - 2));
-      b[i] = *reinterpret_cast<const bf16x8*>(a.w16 + static_cast<int64_t>(n0 + r) * g.K + col);
-    }
-  }
-  __device__ __forceinline__ void store(__bf16* Bs, int S) const {
-#pragma unroll
-    for (int i = 0; i < CHUNKS; ++i) {
-      const int id = threadIdx.x + i * kThreads;
-      *reinterpret_cast<bf16x8*>(Bs + (id >> 2) * S + 8 * (id & 3)) = b[i];
-    }
-  }
-};
-
-// MFMAs of one K step: the wave's columns [wave*TNW*16, +TNW*16) of all four
-// 16-row tiles (W tile first operand: the swapped accumulator layout).
-template <int MATH, int TNW, int RT>
-__device__ __forceinline__ void mma_step_pp(const typename Op<MATH>::T* As, const typename Op<MATH>::T* Bs, int wave,
-                                            int lane, f32x4 (&acc)[RT][TNW]) {
-  constexpr int S = lds_stride<MATH>();
+// fp32 MFMAs of one K step: the wave's columns [wave*TNW*16, +TNW*16) of all
+// four 16-row tiles (W tile first operand: the swapped accumulator layout).
+template <int TNW, int RT>
+__device__ __forceinline__ void mma_step_pp(const float* As, const float* Bs, int wave, int lane,
+                                            f32x4 (&acc)[RT][TNW]) {
+  constexpr int S = lds_stride<kMathF32>();
   const int rl = lane & 15, ks = lane >> 4;
   const int nb = wave * TNW * 16;
-  if constexpr (MATH == kMathBF16) {
-    bf16x8 a[RT];
 #pragma unroll
-    for (int r = 0; r < RT; ++r) a[r] = *reinterpret_cast<const bf16x8*>(As + (16 * r + rl) * S + ks * 8);
+  for (int hk = 0; hk < kBK; hk += 16) {
+    float4 a[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) a[r] = *reinterpret_cast<const float4*>(As + (16 * r + rl) * S + hk + ks * 4);
 #pragma unroll
     for (int f = 0; f < TNW; ++f) {
-      const bf16x8 b = *reinterpret_cast<const bf16x8*>(Bs + (nb + 16 * f + rl) * S + ks * 8);
+      const float4 b = *reinterpret_cast<const float4*>(Bs + (nb + 16 * f + rl) * S + hk + ks * 4);
 #pragma unroll
-      for (int r = 0; r < RT; ++r) mma_bf16<kLdsAsm>(acc[r][f], b, a[r]);
-    }
-  } else {
-#pragma unroll
-    for (int hk = 0; hk < kBK; hk += 16) {
-      float4 a[RT];
-#pragma unroll
-      for (int r = 0; r < RT; ++r) a[r] = *reinterpret_cast<const float4*>(As + (16 * r + rl) * S + hk + ks * 4);
-#pragma unroll
-      for (int f = 0; f < TNW; ++f) {
-        const float4 b = *reinterpret_cast<const float4*>(Bs + (nb + 16 * f + rl) * S + hk + ks * 4);
-#pragma unroll
-        for (int r = 0; r < RT; ++r) mma_f32x4<kLdsAsm>(acc[r][f], b, a[r]);
-      }
+      for (int r = 0; r < RT; ++r) mma_f32x4<kLdsAsm>(acc[r][f], b, a[r]);
     }
   }
 }
 
-// g = G Wp^T + bp and the gamma epilogue; a workgroup owns BM rows and BN of
-// the D outputs (each wavefront BN/4 of them); the next K step's rows and W
-// tile load while the current one runs. With BN < D the D/BN workgroups of a
+// g = G Wp^T + bp and the gamma epilogue with fp32 math; a workgroup owns 64
+// rows and BN of the D outputs (each wavefront BN/4 of them); the next K step's
+// rows and W tile load while the current one runs. With BN < D the D/BN workgroups of a
 // row tile each build its G tiles: with one workgroup per 64 rows, c2's 383
 // workgroups left the GPU at 1.5 wavefronts per SIMD, too few to cover each
 // K step's load latency. One-dimensional grid of 8 ceil(row_tiles / 8) x
@@ -2418,14 +2381,14 @@ __device__ __forceinline__ void mma_step_pp(const typename Op<MATH>::T* As, cons
 // another (ids go round-robin over the 8 XCDs), so they share its rows in L2.
 // The host checks D in {64, 128, 256}, K <= kPackMaxHops, 16-byte aligned
 // rows (H, C, hops, Wp, g_out, h, out).
-template <int MATH, int BN, int BM>
+template <int BN>
 __global__ __launch_bounds__(kThreads) void pack_proj_fwd_kernel(GemmArgs g, PackArgs a, int row_tiles) {
-  using T = typename Op<MATH>::T;
-  constexpr int S = lds_stride<MATH>();
+  constexpr int BM = kPpBM;
+  constexpr int S = lds_stride<kMathF32>();
   constexpr int TNW = BN / 64;
   constexpr int RT = BM / 16;
-  __shared__ __align__(16) T As[2][BM * S];
-  __shared__ __align__(16) T Bs[2][BN * S];
+  __shared__ __align__(16) float As[2][BM * S];
+  __shared__ __align__(16) float Bs[2][BN * S];
   const int ncb = a.D / BN;
   const int xcd = blockIdx.x % 8, jw = blockIdx.x / 8;
   const int rt = (jw / ncb) * 8 + xcd;
@@ -2445,7 +2408,7 @@ __global__ __launch_bounds__(kThreads) void pack_proj_fwd_kernel(GemmArgs g, Pac
   const int jq = a.D / 16;
   const int steps = a.K * jq;
   PackAStage<BM> pa;
-  PackBStage<MATH, BN> pb;
+  PackBStage<BN> pb;
   pa.load(a, m0, 0, 0);
   pb.load(g, a, 0, 0, a.D, n0);
   pa.store(As[0], S, a.mode);
@@ -2459,7 +2422,7 @@ __global__ __launch_bounds__(kThreads) void pack_proj_fwd_kernel(GemmArgs g, Pac
       pa.load(a, m0, kk, j0);
       pb.load(g, a, kk, j0, a.D, n0);
     }
-    mma_step_pp<MATH, TNW, RT>(As[buf], Bs[buf], wave, lane, acc);
+    mma_step_pp<TNW, RT>(As[buf], Bs[buf], wave, lane, acc);
     if (more) {
       pa.store(As[buf ^ 1], S, a.mode);
       pb.store(Bs[buf ^ 1], S);
@@ -2471,11 +2434,153 @@ __global__ __launch_bounds__(kThreads) void pack_proj_fwd_kernel(GemmArgs g, Pac
   epilogue_swapped<kEpiGamma, TNW, RT>(g, acc, m0, n0 + wave * TNW * 16, lane);
 }
 
-// dst[i] = bf16(src[i]) (round to nearest even, as the MFMA operand stores)
-__global__ void to_bf16_kernel(const float* src, int64_t n, __bf16* dst) {
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += static_cast<int64_t>(gridDim.x) * blockDim.x)
-    dst[i] = static_cast<__bf16>(src[i]);
+// ---- forward, bf16 math -------------------------------------------------------
+// Wp in the order pack_proj_fwd16_kernel's lanes read it, rounded to bf16: for
+// K step s (channels 32 (s / K) ..+31, hop s % K), half (W, D) and
+// 16-output tile, the 64 lanes' eight values one after another (lane: output
+// lane % 16, channels 8 (lane / 16) ..+7).
+__global__ void pack_w16_kernel(const float* w, int D, int K, __bf16* dst) {
+  const int64_t chunks = 2LL * K * D * D / 8;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < chunks;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const int lane = static_cast<int>(i & 63);
+    int64_t t = i >> 6;
+    const int nt = static_cast<int>(t % (D / 16));
+    t /= D / 16;
+    const int half = static_cast<int>(t & 1);
+    const int s = static_cast<int>(t >> 1);
+    const int kk = s % K, jb = s / K;
+    const float* p = w + static_cast<int64_t>(nt * 16 + (lane & 15)) * 2 * K * D + kk * 2 * D + half * D + jb * 32 +
+                     (lane >> 4) * 8;
+    float lo[4], hi[4];
+    gload_fast<float, 4>(p, 0, lo);
+    gload_fast<float, 4>(p, 4, hi);
+    bf16x8 v;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      v[q] = static_cast<__bf16>(lo[q]);
+      v[4 + q] = static_cast<__bf16>(hi[q]);
+    }
+    *reinterpret_cast<bf16x8*>(dst + i * 8) = v;
+  }
+}
+
+// g = G Wp^T + bp and the gamma epilogue with bf16 math. A workgroup owns 64
+// rows and all D outputs (each wavefront D/4 of them), K steps of one hop's 32
+// channels: 32 W values, then 32 D values a row, built from H, C and the hop's
+// two halves into LDS, where the four wavefronts read them as MFMA operands.
+// Wp's operands are each wavefront's own, so they go from memory to registers,
+// 1 KB a load (pack_w16_kernel's order).
+//
+// What bounds it is the cache lines a CU asks for (about 8 clocks each, as in
+// the gather kernels) and, with one workgroup on a CU, the chain of a step's
+// products and packing. With 16 channels a step (64-byte pieces of H, C and the
+// hop) and Wp staged through LDS in its own layout (32-byte pieces) a row tile
+// asked for 1,536 pieces per 64 columns of G; here it is 512 lines, the rows
+// are loaded two steps ahead, and the hops follow each other within a channel
+// block, so that H and C come from L2 for all but the first. 24,492 rows, D =
+// 256, K = 3: 107 -> 76 us (83 with the hops outermost and rows one step
+// ahead); whole calls, 2,000 rows 59 -> 40, 11,003 69 -> 46, 60,000 266 -> 197,
+// D = 128 45 -> 36, D = 64 22 -> 20. 96 rows a workgroup: 90 against 92 at
+// 24,492 rows, 67 against 46 at 11,003.
+template <int D, int MODE>
+__global__ __launch_bounds__(kThreads, 2) void pack_proj_fwd16_kernel(GemmArgs g, PackArgs a) {
+  constexpr int TNW = D / 64;
+  constexpr int BM = kPpBM;
+  constexpr int RT = BM / 16;
+  constexpr int NP = BM / 32;  // rows of a thread
+  constexpr int S = 40;  // LDS row stride: 32 values and 16 bytes
+  constexpr int JB = D / 32;
+  __shared__ __align__(16) __bf16 As[2][2][BM * S];  // buffer, half
+  const int lane = lane_id();
+  const int wave = wave_id();
+  const int rl = lane & 15, ks = lane >> 4;
+  const int64_t m0 = static_cast<int64_t>(blockIdx.x) * BM;
+  const int steps = a.K * JB;  // even: JB is
+
+  // The thread's part of a step's rows: rows tr, tr + 32, ..., four channels.
+  const int tr = threadIdx.x >> 3, tc = 4 * (threadIdx.x & 7);
+  int64_t mr[NP];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) mr[p] = min(m0 + tr + 32 * p, a.M - 1);  // rows past M: outputs never stored
+  struct Rows {
+    float hv[NP][4], cv[NP][4], ph[NP][4], pc[NP][4], al[NP];
+  };
+  const auto load_rows = [&](int s, Rows& x) {
+    const int kk = s % a.K, j = (s / a.K) * 32 + tc;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      gload_fast<float, 4>(a.H + mr[p] * D, j, x.hv[p]);
+      gload_fast<float, 4>(a.C + mr[p] * D, j, x.cv[p]);
+      const float* pk = a.P[kk] + mr[p] * a.p_stride;
+      gload_fast<float, 4>(pk, j, x.ph[p]);
+      gload_fast<float, 4>(pk, D + j, x.pc[p]);
+      x.al[p] = a.alpha[mr[p] * a.a_stride + kk];
+    }
+  };
+  const auto store_rows = [&](int buf, const Rows& x) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      float w[4], d[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const packk::DW e = packk::interact(x.hv[p][q] * x.pc[p][q], x.cv[p][q] * x.ph[p][q], MODE);
+        w[q] = x.al[p] * e.Wv;
+        d[q] = x.al[p] * e.Dv;
+      }
+      st_lds<__bf16, 4>(As[buf][0] + (tr + 32 * p) * S + tc, w);
+      st_lds<__bf16, 4>(As[buf][1] + (tr + 32 * p) * S + tc, d);
+    }
+  };
+  const __bf16* wl = a.w16 + (static_cast<int64_t>(wave) * TNW * 64 + lane) * 8;
+  const auto load_w = [&](int s, bf16x8 (&wb)[2][TNW]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int f = 0; f < TNW; ++f)
+        wb[h][f] = *reinterpret_cast<const bf16x8*>(wl + ((2LL * s + h) * (D / 16) + f) * 512);
+  };
+
+  f32x4 acc[RT][TNW];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int f = 0; f < TNW; ++f) acc[r][f] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  if constexpr (kLdsAsm) mfma_settle(acc);
+  bf16x8 wb[2][2][TNW];
+  Rows x[2];
+  load_rows(0, x[0]);
+  load_w(0, wb[0]);
+  load_rows(min(1, steps - 1), x[1]);
+  store_rows(0, x[0]);
+  __syncthreads();
+  // One step: the rows of the step after the next, then the next one's W
+  // operands, in flight during this one's products and the packing of the next
+  // one's rows. Past the end the last step is loaded again.
+  const auto step = [&](int s, int buf, bf16x8 (&cur)[2][TNW], bf16x8 (&nxt)[2][TNW], Rows& next, Rows& after) {
+    load_w(min(s + 1, steps - 1), nxt);
+    load_rows(min(s + 2, steps - 1), after);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      bf16x8 av[RT];
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+        av[r] = *reinterpret_cast<const bf16x8*>(As[buf][h] + (16 * r + rl) * S + ks * 8);
+#pragma unroll
+      for (int f = 0; f < TNW; ++f)
+#pragma unroll
+        for (int r = 0; r < RT; ++r) mma_bf16<kLdsAsm>(acc[r][f], cur[h][f], av[r]);
+    }
+    store_rows(buf ^ 1, next);
+    __syncthreads();
+  };
+  for (int s = 0; s < steps; s += 2) {
+    step(s, 0, wb[0], wb[1], x[1], x[0]);
+    step(s + 1, 1, wb[1], wb[0], x[0], x[1]);
+  }
+  if constexpr (kLdsAsm) mfma_settle(acc);
+  epilogue_swapped<kEpiGamma, TNW, RT>(g, acc, m0, wave * TNW * 16, lane);
 }
 
 // ---- backward: grad_G and the pack's backward --------------------------------
@@ -3431,35 +3536,33 @@ int cign_pack_proj_fwd(void* stream, int64_t n, int32_t D, int32_t K, int32_t in
   g.h = h; g.gamma = gamma; g.p = dropout_p; g.seed = seed; g.out = out; g.mask = mask;
   PackArgs a = pp_args(n, D, K, interaction, H, C, props, prop_stride, alpha, alpha_stride);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const int row_tiles = static_cast<int>((n + kPpBM - 1) / kPpBM);
   if (math == kMathBF16) {
     __bf16* w16 = static_cast<__bf16*>(workspace);
-    const int64_t nw = 2LL * K * D * D;
-    hipLaunchKernelGGL(to_bf16_kernel, dim3(static_cast<unsigned>(std::min<int64_t>((nw + 255) / 256, 2048))),
-                       dim3(256), 0, st, w, nw, w16);
+    const int64_t chunks = 2LL * K * D * D / 8;
+    hipLaunchKernelGGL(pack_w16_kernel, dim3(static_cast<unsigned>(std::min<int64_t>((chunks + 255) / 256, 2048))),
+                       dim3(256), 0, st, w, D, K, w16);
     if ((rc = check_launch("cign_pack_proj_fwd (bf16 weight)"))) return rc;
     a.w16 = w16;
-  }
-  // 64-row tiles: at the c2 block (24.5K rows, D = 256, bf16) 119 us against
-  // 146 us with 32-row tiles (twice the workgroups, twice the W tile loads)
-  auto go = [&](auto MC) {
-    constexpr int M_ = decltype(MC)::value;
-    const int row_tiles = static_cast<int>((n + kPpBM - 1) / kPpBM);
-    auto launch = [&](auto BNC) {
-      constexpr int BN = decltype(BNC)::value;
-      const dim3 grid1(static_cast<unsigned>((row_tiles + 7) / 8 * 8 * (D / BN)));
-      hipLaunchKernelGGL((pack_proj_fwd_kernel<M_, BN, kPpBM>), grid1, dim3(kThreads), 0, st, g, a, row_tiles);
+    auto launch = [&](auto DC, auto MC) {
+      hipLaunchKernelGGL((pack_proj_fwd16_kernel<decltype(DC)::value, decltype(MC)::value>),
+                         dim3(static_cast<unsigned>(row_tiles)), dim3(kThreads), 0, st, g, a);
     };
-    // Column block: all D outputs with bf16 math (at the production block
-    // 120 us against 122 us with 128 and 153 us with 64), 64 with fp32 math,
-    // whose double-buffered fp32 tiles of all 256 outputs took 92 KB of LDS
-    // and one workgroup per CU (229 us against 237 us with 128 and 317 us
-    // with 256).
-    if (D == 64 || M_ == kMathF32) launch(std::integral_constant<int, 64>());
-    else if (D == 128) launch(std::integral_constant<int, 128>());
-    else launch(std::integral_constant<int, 256>());
-  };
-  if (math == kMathBF16) go(std::integral_constant<int, kMathBF16>());
-  else go(std::integral_constant<int, kMathF32>());
+    auto modes = [&](auto DC) {
+      if (a.mode == 0) launch(DC, std::integral_constant<int, 0>());
+      else if (a.mode == 1) launch(DC, std::integral_constant<int, 1>());
+      else launch(DC, std::integral_constant<int, 2>());
+    };
+    if (D == 64) modes(std::integral_constant<int, 64>());
+    else if (D == 128) modes(std::integral_constant<int, 128>());
+    else modes(std::integral_constant<int, 256>());
+  } else {
+    // 64 of the D outputs a workgroup: its double-buffered fp32 tiles of all
+    // 256 outputs took 92 KB of LDS and one workgroup per CU (229 us against
+    // 237 us with 128 outputs and 317 us with 256).
+    const dim3 grid1(static_cast<unsigned>((row_tiles + 7) / 8 * 8 * (D / 64)));
+    hipLaunchKernelGGL((pack_proj_fwd_kernel<64>), grid1, dim3(kThreads), 0, st, g, a, row_tiles);
+  }
   return check_launch(who);
 }
 

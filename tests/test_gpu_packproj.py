@@ -187,3 +187,12 @@ def test_pack_proj_rejects_bad_shapes():
     assert lib.cign_pack_proj_bwd_workspace_bytes(100, 48, 3) == 0
     assert lib.cign_pack_proj_fwd_workspace_bytes(256, 3, 0) == 0
     assert lib.cign_pack_proj_fwd_workspace_bytes(256, 3, 1) == 2 * 256 * 6 * 256
+
+
+@pytest.mark.parametrize("n,D,K,interaction", [(1, 128, 1, 0), (63, 256, 2, 0), (64, 128, 2, 2), (65, 128, 3, 1),
+                                               (129, 64, 4, 2), (200, 256, 4, 1)])
+def test_pack_proj_bf16_row_tiles(n, D, K, interaction):
+    """The bf16 forward's row tiles (one row, one short of a tile, a whole
+    one, one over) at each width, hop count and interaction it is compiled
+    for."""
+    test_pack_proj_matches_oracle(n, D, K, interaction, "node", "new", True)
