@@ -1289,10 +1289,31 @@ __device__ __forceinline__ bool wg_tile_chunk(int tiles, int chunks, bool xcd, i
 inline unsigned wg_grid(int tiles, int chunks, bool xcd) {
   return static_cast<unsigned>(tiles * (xcd ? (chunks + 7) / 8 * 8 : chunks));
 }
-// Row chunks of those kernels: about `target`; with `xcd` a multiple of 8
-// (one per XCD each round) once there are at least 8.
-inline int64_t wg_chunk_count(int64_t M, int64_t target, bool xcd) {
-  const int64_t c = std::max<int64_t>(1, std::min<int64_t>((M + 255) / 256, target));
+// Row chunks of those kernels: 512 workgroups over the tiles at most, and
+// chunks of at least 128 rows (4 k-steps of kWgM: fewer spend longer filling
+// the pipeline and on the partials than the extra workgroups save), or 64
+// where even so fewer than 64 workgroups run. With bf16 operands 256 rows
+// where that already gives each CU a workgroup. The launches are latency
+// bound while the chip is short of workgroups; fixed 256-row chunks against
+// this rule, with the partials' sum, us:
+//   grad_W fp32  2,000 x 256 x 64: 30.4, 13.9    5,000 x 256 x 128: 27.4, 19.7
+//                1,200 x 512 x 300: 30.4, 22.8   11,003 x 480 x 96: 38.0, 34.9
+//                24,492 x 192 x 192: 51.7, 43.8
+//   grad_W bf16  2,000 x 256 x 64: 17.4, 10.8    11,003 x 96 x 576: 24.7, 22.0
+//   pack projection's backward, D x K, fp32
+//                2,000 x 64 x 2: 62.0, 41.8      24,492 x 64 x 3: 112.6, 100.8
+//   the same in bf16 at 11,003 x 128 x 3 (258 workgroups of 256 rows): 90.4
+//   with 256-row chunks, 98.3 with 128: twice the partials for one more round
+//   of a chip that has one already; so bf16 keeps 256 there.
+// Chunks of 32 rows were slower than 64 from 64 workgroups on (5,000 x 256 x
+// 128: 21.3 against 17.3 with 64). With `xcd` a multiple of 8 chunks (one per
+// XCD each round) once there are at least 8.
+inline int64_t wg_chunk_count(int64_t M, int64_t tiles, bool xcd) {
+  const auto by = [&](int64_t rows) { return (M + rows - 1) / rows; };
+  int64_t rows = 128;
+  if (xcd && tiles * by(256) >= 256) rows = 256;
+  else if (tiles * by(128) < 64) rows = 64;
+  const int64_t c = std::max<int64_t>(1, std::min<int64_t>(by(rows), std::max<int64_t>(1, 512 / tiles)));
   return xcd && c >= 8 ? (c + 7) / 8 * 8 : c;
 }
 
@@ -3066,9 +3087,9 @@ struct BwdWs {
   int64_t chunk, wg_chunk, part_b, part_w, wt, total;
 };
 
-// xcd: the chunking of bf16 operands (wg_tile_chunk); the workspace size
-// query takes it (the larger layout) for either math.
-inline BwdWs bwd_ws(int64_t M, int N, int K, bool bias, bool xcd = true) {
+// xcd: the chunking of bf16 operands (wg_tile_chunk). Either math may have
+// the more chunks; the workspace size query takes the larger layout.
+inline BwdWs bwd_ws(int64_t M, int N, int K, bool bias, bool xcd) {
   BwdWs L;
   // row chunks of the bias (and, for few outputs, grad_W) partials: 64 rows,
   // or 16 for few outputs (more workgroups for the per-chunk VALU sums)
@@ -3081,8 +3102,8 @@ inline BwdWs bwd_ws(int64_t M, int N, int K, bool bias, bool xcd = true) {
   int64_t off = 0;
   L.part_b = off; off = al(off + (bias ? 4LL * chunks * N : 0));
   // grad_W partials per row chunk: the few-output VALU sums use the bias
-  // chunks; the MFMA kernel takes chunks of >= 256 rows, about 512
-  // workgroups over its 128 x 128 tiles
+  // chunks; the MFMA kernel takes the row chunks of wg_chunk_count over its
+  // 128 x 128 tiles
   const bool small = N <= kSmallN;
   if (!small && N <= kNarrowN) {
     // wgrad_narrow_kernel: 64-wide k tiles, chunks of a multiple of 64 rows
@@ -3091,7 +3112,7 @@ inline BwdWs bwd_ws(int64_t M, int N, int K, bool bias, bool xcd = true) {
     const int64_t ntk = (K + kWnK - 1) / kWnK;
     // (about 512: fewer workgroups left the chip short, more spent longer
     // on the chunk partials and their sums than they saved, at the c2 lin)
-    int64_t wgc = wg_chunk_count(M, std::max<int64_t>(1, 512 / ntk), true);
+    int64_t wgc = wg_chunk_count(M, ntk, true);
     L.wg_chunk = std::max<int64_t>(kWnChunkRows,
                                    ((M + wgc - 1) / wgc + kWnChunkRows - 1) / kWnChunkRows * kWnChunkRows);
     wgc = M > 0 ? (M + L.wg_chunk - 1) / L.wg_chunk : 1;
@@ -3102,7 +3123,7 @@ inline BwdWs bwd_ws(int64_t M, int N, int K, bool bias, bool xcd = true) {
     return L;
   }
   const int64_t tiles = static_cast<int64_t>((N + kWgT - 1) / kWgT) * ((K + kWgT - 1) / kWgT);
-  int64_t wgc = wg_chunk_count(M, std::max<int64_t>(1, 512 / tiles), xcd);
+  int64_t wgc = wg_chunk_count(M, tiles, xcd);
   L.wg_chunk = std::max<int64_t>(kWgM, ((M + wgc - 1) / wgc + kWgM - 1) / kWgM * kWgM);
   wgc = M > 0 ? (M + L.wg_chunk - 1) / L.wg_chunk : 1;
   L.wg_chunks = static_cast<int>(wgc);
@@ -3125,12 +3146,12 @@ struct PpWs {
 
 inline int pp_ntk(int D, int K) { return K * (D / 64); }
 
-inline PpWs pp_ws(int64_t M, int D, int K, bool xcd = true) {
+inline PpWs pp_ws(int64_t M, int D, int K, bool xcd) {
   PpWs L;
   auto al = [](int64_t v) { return (v + 255) & ~int64_t(255); };
   const int64_t kw = 2LL * K * D;
   const int64_t tiles = static_cast<int64_t>((D + kWgT - 1) / kWgT) * pp_ntk(D, K);
-  int64_t wgc = wg_chunk_count(M, std::max<int64_t>(1, 512 / tiles), xcd);
+  int64_t wgc = wg_chunk_count(M, tiles, xcd);
   L.wg_chunk = std::max<int64_t>(kWgM, ((M + wgc - 1) / wgc + kWgM - 1) / kWgM * kWgM);
   L.wg_chunks = static_cast<int>(M > 0 ? (M + L.wg_chunk - 1) / L.wg_chunk : 1);
   int64_t bc = std::max<int64_t>(1, std::min<int64_t>(1024, (M + 63) / 64));
@@ -3279,7 +3300,7 @@ int cign_linear_gamma_fwd(void* stream, int64_t M, int32_t N, int32_t K, int32_t
 }
 
 int64_t cign_linear_bwd_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t with_bias) {
-  return bwd_ws(M, N, K, with_bias != 0).total;
+  return std::max(bwd_ws(M, N, K, with_bias != 0, true).total, bwd_ws(M, N, K, with_bias != 0, false).total);
 }
 
 // Row chunks of cign_lin_logits_wgrad (wgrad_narrow_kernel's) and its
@@ -3293,7 +3314,7 @@ struct WlWs {
 inline WlWs wl_ws(int64_t M, int N, int K) {
   WlWs L;
   L.ntk = (K + kWnK - 1) / kWnK;
-  int64_t wgc = wg_chunk_count(M, std::max<int64_t>(1, 512 / L.ntk), true);
+  int64_t wgc = wg_chunk_count(M, L.ntk, true);
   L.chunk = std::max<int64_t>(kWnChunkRows, ((M + wgc - 1) / wgc + kWnChunkRows - 1) / kWnChunkRows * kWnChunkRows);
   wgc = M > 0 ? (M + L.chunk - 1) / L.chunk : 1;
   L.chunks = static_cast<int>(wgc);
@@ -3568,7 +3589,7 @@ int cign_pack_proj_fwd(void* stream, int64_t n, int32_t D, int32_t K, int32_t in
 
 int64_t cign_pack_proj_bwd_workspace_bytes(int64_t n, int32_t D, int32_t K) {
   if (n < 0 || K < 1 || K > kPackMaxHops || (D != 64 && D != 128 && D != 256)) return 0;
-  return pp_ws(n, D, K).total;
+  return std::max(pp_ws(n, D, K, true).total, pp_ws(n, D, K, false).total);
 }
 
 int cign_pack_proj_bwd(void* stream, int64_t n, int32_t D, int32_t K, int32_t interaction, int32_t math,

@@ -85,6 +85,30 @@ def _check_amp_backward(gy, x, w, gx, gw, gb):
         assert_bf16_sum_close(gb, eb, np.abs(gyr).sum(0), M, "grad_b (amp)")
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (1, 256, 64), (63, 256, 64), (65, 256, 64), (2000, 256, 64),  # 64-row chunks
+    (3968, 256, 64), (3969, 256, 64),  # 2 tiles: 64 rows up to 31 chunks of 128, then 128
+    (1792, 512, 1024), (1793, 512, 1024),  # 32 tiles, bf16: 256 rows once 8 such chunks
+    (511, 64, 256), (1920, 64, 256), (1921, 64, 256),  # the narrow kernel, 4 tiles
+])
+@pytest.mark.parametrize("amp", [False, True])
+def test_weight_gradient_row_chunks(M, N, K, amp):
+    """grad_W over every row of its chunks, once. Whole operands in [-2, 2]:
+    products and sums up to 4 M are exact in fp32, so the fp32 result equals
+    the integer product, the bf16 one its rounding."""
+    from cign_amd.linear import mfma_linear
+
+    print(f"wgrad chunks M={M} N={N} K={K} amp={amp}", flush=True)
+    g = torch.Generator().manual_seed(M + N)
+    x = torch.randint(-2, 3, (M, K), generator=g).float()
+    gy = torch.randint(-2, 3, (M, N), generator=g).float()
+    ref = gy.double().T @ x.double()
+    lin = nn.Linear(K, N).cuda()
+    mfma_linear(lin, x.cuda().requires_grad_(True), amp).backward(gy.cuda())
+    ref = ref.to(torch.bfloat16).float() if amp else ref.float()
+    assert torch.equal(lin.weight.grad.cpu(), ref)
+
+
 def test_linear_bf16_input():
     from cign_amd.linear import mfma_linear
 
