@@ -202,6 +202,12 @@ inline void gat_geometry(int pass, int dtype, int H, int C, int& light, int& seg
   }
 }
 
+// Whether a schedule of a padded shape has the pair layout's geometry: one
+// that was built (or stored) for that layout keeps running it.
+inline bool pair_sched(int dtype, int H, int C, const int32_t* info) {
+  return info && info[3] == kGatSeg && info[4] == kGatLight && fl_ok(dtype, H, C) && !fl_exact(dtype, H, C);
+}
+
 // Host view of a schedule header (schedule.h).
 struct Hdr {
   int n_light, n_seg, n_hrow;
@@ -274,6 +280,8 @@ int gat_fwd_impl(void* stream, int32_t dtype, int32_t n, int32_t nnz, int32_t he
   Hdr hd;
   int light, seg;
   gat_geometry(0, dtype, heads, channels, light, seg);
+  const bool pair = pair_sched(dtype, heads, channels, row_sched_info);
+  if (pair) light = kGatLight, seg = kGatSeg;
   if ((rc = read_hdr("cign_gat_fwd", row_sched_info, n, light, seg, hd))) return rc;
   if (workspace_bytes < cign_gat_fwd_workspace_bytes(hd.n_seg, heads, channels))
     return set_error(kInvalid, "cign_gat_fwd: workspace too small");
@@ -295,7 +303,7 @@ int gat_fwd_impl(void* stream, int32_t dtype, int32_t n, int32_t nnz, int32_t he
     a.agg = row_agg;
     int L, V;
     bool exact;
-    if (fl_geom_w(FlGeom<T>::W, heads, channels, L, V, exact) && (exact || !std::is_same_v<T, bf16x>)) {
+    if (!pair && fl_geom_w(FlGeom<T>::W, heads, channels, L, V, exact) && (exact || !std::is_same_v<T, bf16x>)) {
       if (exact && (!aligned16(xt) || !aligned16(ot) || !aligned16(pre)))
         return set_error(kInvalid, "cign_gat_fwd: in_feat, out and pre must be 16-byte aligned");
       const int lgcq = fl_lgcq_w(FlGeom<T>::W, channels);
@@ -312,7 +320,7 @@ int gat_fwd_impl(void* stream, int32_t dtype, int32_t n, int32_t nnz, int32_t he
     else return dispatch_hc<FwdLauncher, T>(heads, channels, st, a, s);
   };
   if (dtype == kF32) return fill(static_cast<const float*>(in_feat), static_cast<float*>(out));
-  if (dtype == kBF16 && fl_half(dtype, heads, channels, graph_nnz))
+  if (dtype == kBF16 && !pair && fl_half(dtype, heads, channels, graph_nnz))
     return fill(static_cast<const bf16h*>(in_feat), static_cast<bf16h*>(out));
   if (dtype == kBF16) return fill(static_cast<const bf16*>(in_feat), static_cast<bf16*>(out));
   if (dtype == kBF16F32) return fill(static_cast<const bf16x*>(in_feat), static_cast<float*>(out));
@@ -378,6 +386,10 @@ int gat_bwd_impl(void* stream, int32_t dtype, int32_t n, int32_t nnz, int32_t he
   Hdr rh, ch;
   int light, seg;
   gat_geometry(1, dtype, heads, channels, light, seg);
+  const bool pair = pair_sched(dtype, heads, channels, row_sched_info);
+  if (pair && att_src)
+    return set_error(kInvalid, "cign_gat_bwd_logits: schedules of the pair layout (cign_gat_schedule_params)");
+  if (pair) light = kGatLight, seg = kGatSeg;
   if ((rc = read_hdr("cign_gat_bwd (rows)", row_sched_info, n, light, seg, rh))) return rc;
   if ((rc = read_hdr("cign_gat_bwd (cols)", col_sched_info, n, light, seg, ch))) return rc;
   const Sched rs = make_sched(row_sched, rh.n_light, rh.n_seg, rh.n_hrow);
@@ -418,7 +430,7 @@ int gat_bwd_impl(void* stream, int32_t dtype, int32_t n, int32_t nnz, int32_t he
     a.grad_feat = gxt; a.grad_attn_row = grad_attn_row; a.grad_attn_col = grad_attn_col; a.grad_bias = grad_bias;
     int FL, FV;
     bool exact;
-    if (fl_geom_w(FlGeom<T>::W, heads, channels, FL, FV, exact) && (exact || !std::is_same_v<T, bf16x>)) {
+    if (!pair && fl_geom_w(FlGeom<T>::W, heads, channels, FL, FV, exact) && (exact || !std::is_same_v<T, bf16x>)) {
       if (exact &&
           (!aligned16(xt) || !aligned16(gyt) || !aligned16(gxt) || !aligned16(pre) || !aligned16(grad_bias)))
         return set_error(kInvalid, "cign_gat_bwd: in_feat, pre, grad_y, grad_feat and grad_bias must be 16-byte "
@@ -447,7 +459,7 @@ int gat_bwd_impl(void* stream, int32_t dtype, int32_t n, int32_t nnz, int32_t he
   };
   if (dtype == kF32)
     return fill(static_cast<const float*>(in_feat), static_cast<const float*>(grad_y), static_cast<float*>(grad_feat));
-  if (dtype == kBF16 && fl_half(dtype, heads, channels, graph_nnz))
+  if (dtype == kBF16 && !pair && fl_half(dtype, heads, channels, graph_nnz))
     return fill(static_cast<const bf16h*>(in_feat), static_cast<const bf16h*>(grad_y), static_cast<bf16h*>(grad_feat));
   if (dtype == kBF16)
     return fill(static_cast<const bf16*>(in_feat), static_cast<const bf16*>(grad_y), static_cast<bf16*>(grad_feat));

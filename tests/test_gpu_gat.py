@@ -424,3 +424,17 @@ def test_padded_heads_unaligned_tensors(H, C, dtype):
     assert torch.equal(out, out2)
     for a, e in zip(grads2, grads):
         assert torch.equal(a, e)
+
+
+@pytest.mark.parametrize("H,C,dtype", [(5, 48, torch.float32), (3, 100, torch.float32), (5, 24, torch.bfloat16),
+                                       (6, 96, torch.bfloat16)])
+def test_padded_heads_take_pair_layout_schedules(H, C, dtype, monkeypatch):
+    """Schedules of the pair layout's geometry (16 light edges, 64-edge
+    segments) run the pair layout on the padded shapes, forward and backward;
+    on the others they are refused."""
+    from cign_amd import schedule
+
+    monkeypatch.setattr(schedule, "_gat_params", lambda pass_, code, heads, channels: (16, 64))
+    test_ext_forward_backward_matches_oracle(H, C, 0.5, dtype, 300, {0: 700, 5: 90}, True, False, monkeypatch)
+    with pytest.raises(RuntimeError, match="light_max"):
+        test_ext_forward_backward_matches_oracle(4, 16, 0.0, dtype, 300, {0: 700}, True, False, monkeypatch)
