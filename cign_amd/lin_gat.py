@@ -6,8 +6,10 @@ The reference runs three functions: ``_local_amp_linear`` (the ``lin``,
 model_cign.py:86-103), the attention logits (fused_gat_sideops.py:94-97) and
 the collapsed GAT (collapsed_gat.py:164-225). x_proj feeds both the logits
 and the GAT, so autograd sums their two gradients of it in a pass of its own
-before the projection's backward; here the logits' backward adds the GAT's
-gradient as it writes its own (cign_attn_logits_bwd_acc), which is that sum.
+before the projection's backward; here the GAT's columns pass adds the
+logits' terms as it writes its own gradient (cign_gat_bwd_logits), or, on
+the shapes and graphs that does not take, the logits' backward adds the
+GAT's gradient as it writes its own (cign_attn_logits_bwd_acc): that sum.
 
 Under selective bf16 AMP the ``lin`` returns ``.float()`` of a bf16 result,
 so x_proj holds bf16 values. Where the library runs the GAT on bf16 features
@@ -16,7 +18,7 @@ projection stores those values as bf16 and every consumer reads them so
 with fp32 math: the forward computes what the fp32 x_proj gives, in half the
 bytes, and the backward rounds where the reference does (the two gradients
 summed in fp32, then rounded to bf16 for the projection's backward, as
-autocast's backward does; the logits' backward stores the sum so rounded,
+autocast's backward does; the kernel that forms the sum stores it so rounded,
 and cign_linear_bwd_bf16gy reads it in half the bytes and returns grad_x and
 grad_W rounded to bf16, the bf16 Linear's backward outputs). That needs one
 function: autograd would round each consumer's gradient to the dtype of a

@@ -106,9 +106,10 @@ int cign_gat_schedule_params(int32_t pass, int32_t dtype, int32_t heads, int32_t
 int64_t cign_gat_fwd_workspace_bytes(int32_t n_seg, int32_t heads, int32_t channels);
 
 /* Floats of the optional per-row aggregate buffer (row_agg) that
- * cign_gat_fwd fills and cign_gat_bwd reads, n*H*(2C+1) for the shapes of
- * the feature-layout kernels (H <= 8, C a multiple of 16 bytes' worth of
- * elements with C/that a power of two, H*C <= 64 such chunks), 0 otherwise.
+ * cign_gat_fwd fills and cign_gat_bwd reads, n*H*(2C+1) for the exact
+ * shapes of the feature-layout kernels (H <= 8, C a multiple of 16 bytes'
+ * worth of elements with C/that a power of two, H*C at most 64 such chunks
+ * or 2, 3, 4, 6 or 8 times 64), 0 otherwise.
  * The buffer holds sum_e s kw x[j], sum_e s kw l' x[j] ([n,H,C] each) and
  * sum_e s l' ([n,H]) per destination row, so the backward need not gather
  * the source rows a second time. No counterpart in the reference: its
