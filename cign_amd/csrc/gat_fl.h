@@ -229,6 +229,16 @@ __device__ __forceinline__ void store_values(T* p, const float (&v)[W]) {
   }
 }
 
+// Index of entry `slot` of the list at p (deg entries from `first`), or for a
+// lane past its end of the list's first entry: the batches read whatever row a
+// lane's index names and give a slot past the end weight 0, so that row has to
+// be one the list's owner reads anyway. (Index 0 there carried a NaN or an
+// infinity of node 0, 0 times it, into nearly every row.) An empty list reads
+// nothing and has index 0; its owner drops what its slots added.
+__device__ __forceinline__ int list_index(const int32_t* p, int first, int deg, int slot) {
+  return deg > 0 ? p[first + (slot < deg ? slot : 0)] : 0;
+}
+
 // Largest value of v over the groups of a wavefront (lane bits >= log2 L).
 template <int L>
 __device__ __forceinline__ int wave_group_max(int v) {
@@ -398,9 +408,9 @@ struct FwdBatches {
     constexpr int NT = (U + R - 1) / R;  // slots whose weights this lane computes
     const uint32_t rowB = static_cast<uint32_t>(a.H * a.C) * sizeof(T);
     typename Chunk<T, W>::Raw xb[U][V];
-    // Slot u's index is held by lane (base + u) mod 64. Every lane holds a
-    // valid column index (0 where it has no edge), so a slot past cnt reads
-    // some valid row, weighted 0, and needs no clamp.
+    // Slot u's index is held by lane (base + u) mod 64. Every lane holds an
+    // index (list_index), so a slot past cnt reads a row of the group's own,
+    // weighted 0, and needs no clamp.
     const int ub = base + first + k0 * step;
 #pragma unroll
     for (int k = 0; k < U; ++k) {
@@ -632,10 +642,11 @@ __global__ __launch_bounds__(kBlock) void gat_fwd_fl_kernel(GatFwdArgs<T> a, Sch
       const bool has = li < s.n_light;
       const int4 r = has ? s.light[li] : make_int4(0, 0, 0, 0);
       const int deg = r.z - r.y;
-      const int jj = ln.gl < deg ? a.col[r.y + ln.gl] : 0;
+      const int jj = list_index(a.col, r.y, deg, ln.gl);
       load_attn_row(a, ln, r.x, ar);
       const int need = wave_group_max<L>(deg);
       fwd_edges<T, L, V, DROP, R, UM>(a, ln, jj, ln.g * L, 0, 1, deg, need, r.y, ar, st);
+      if (deg == 0) st.clear();
       quad_reduce<R>(st);
       fwd_emit<T, L, V>(a, ln, cq, r.x, has, st);
       return;
@@ -646,7 +657,7 @@ __global__ __launch_bounds__(kBlock) void gat_fwd_fl_kernel(GatFwdArgs<T> a, Sch
     if (li >= n_mid) return;  // wave-uniform; no block barrier follows
     const int4 r = s.light[li];
     const int deg = r.z - r.y;
-    const int jj = ln.lane < deg ? a.col[r.y + ln.lane] : 0;
+    const int jj = list_index(a.col, r.y, deg, ln.lane);
     load_attn_row(a, ln, r.x, ar);
     fwd_edges<T, L, V, DROP, R, UM>(a, ln, jj, 0, ln.g, G, deg, (deg + G - 1) / G, r.y, ar, st);
     quad_reduce<R>(st);
@@ -666,11 +677,11 @@ __global__ __launch_bounds__(kBlock) void gat_fwd_fl_kernel(GatFwdArgs<T> a, Sch
   // The next round's column indices are loaded before this round's gathers,
   // so a round waits on one memory latency (the gathers) instead of two.
   int tb = sg.y + wave * kWave;
-  int jj = tb + ln.lane < sg.z ? a.col[tb + ln.lane] : 0;
+  int jj = a.col[min(tb + ln.lane, sg.z - 1)];
   for (; tb < sg.z; tb += kSegRound) {
     const int cnt = min(kWave, sg.z - tb);
     const int tn = tb + kSegRound + ln.lane;
-    const int jn = tn < sg.z ? a.col[tn] : 0;
+    const int jn = tn < sg.z ? a.col[tn] : jj;
     fwd_edges<T, L, V, DROP, R, UM>(a, ln, jj, 0, ln.g, G, cnt, (cnt + G - 1) / G, tb, ar, st);
     jj = jn;
   }
@@ -978,7 +989,7 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_rows_fl_kernel(GatBwdArgs<T> a
     const int row = r.x;
     const int deg = r.z - r.y;
     const int slot = tiny ? ln.gl : ln.lane;
-    const int jj = slot < deg ? a.col[r.y + slot] : 0;
+    const int jj = list_index(a.col, r.y, deg, slot);
     const RowHead<V> rh = row_head(a, row, ln);
     grad_pre_chunk(a, row, ln.cw, gp);
     if (tiny) {
@@ -988,6 +999,9 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_rows_fl_kernel(GatBwdArgs<T> a
       rows_group_sum<L, W, V>(st);
     }
     rows_dots<L, W, V>(ln, st, st.B, gp, cq, a.inv_h, wsum, A);
+    if (deg == 0)
+#pragma unroll
+      for (int v = 0; v < V; ++v) wsum[v] = A[v] = 0.0f;
     if (has && (tiny || ln.g == 0)) rows_emit(a, ln, row, rh, wsum, A, gp);
     return;
   }
@@ -1001,11 +1015,11 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_rows_fl_kernel(GatBwdArgs<T> a
   grad_pre_chunk(a, row, ln.cw, gp);
   // next round's indices loaded before this round's gathers, as in the forward
   int tb = sg.y + wave * kWave;
-  int jj = tb + ln.lane < sg.z ? a.col[tb + ln.lane] : 0;
+  int jj = a.col[min(tb + ln.lane, sg.z - 1)];
   for (; tb < sg.z; tb += kSegRound) {
     const int cnt = min(kWave, sg.z - tb);
     const int tn = tb + kSegRound + ln.lane;
-    const int jn = tn < sg.z ? a.col[tn] : 0;
+    const int jn = tn < sg.z ? a.col[tn] : jj;
     rows_edges<T, L, V, DROP>(a, ln, jj, 0, ln.g, G, cnt, (cnt + G - 1) / G, tb, rh, st);
     jj = jn;
   }
@@ -1125,7 +1139,7 @@ constexpr bool cols_pairwise() {
 
 // Softmax weight e^(leaky(raw) - max) / sum of a CSC entry from its
 // destination row's record rs = {attn_row, max, 1/sum, wsum}; 0 for an unused
-// slot. Branch-free: an unused slot's record (some valid row's) is loaded
+// slot. Branch-free: an unused slot's record (another entry's) is loaded
 // like the others and the selects leave nothing to do conditionally, so the
 // whole record arrives in one 16-byte load instead of a second load issued
 // behind a branch once the first has returned.
@@ -1141,8 +1155,8 @@ __device__ __forceinline__ uint64_t rec_off(uint32_t i, int stride) {
 
 // Batches of CSC entries of column j: slot u's destination row is held by
 // lane (base + u) mod 64 in ii, its CSR edge id (used only with dropout) in
-// ee. Every lane holds a valid row and edge id (0 where it has no entry), so
-// a slot past cnt reads some valid record, weighted 0, without a clamp. The
+// ee. Every lane holds a row and edge id (list_index), so a slot past cnt
+// reads a record of the column's own, weighted 0, without a clamp. The
 // g_pre chunk of a destination row is shared by the lane's V heads.
 template <typename T, int L, int V, bool DROP>
 struct ColBatches {
@@ -1508,9 +1522,8 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_cols_fl_kernel(GatBwdArgs<T> a
     const int j = r.x;
     const int deg = r.z - r.y;
     const int slot = tiny ? ln.gl : ln.lane;
-    const bool own = slot < deg;
-    const int ii = own ? a.rowind[r.y + slot] : 0;
-    const int ee = (DROP && own) ? a.perm[r.y + slot] : 0;
+    const int ii = list_index(a.rowind, r.y, deg, slot);
+    const int ee = DROP ? list_index(a.perm, r.y, deg, slot) : 0;
     load_attn_col(a, ln, j, ac);
     XCol<T, V> xc;
     xc.prefetch(a, ln, j);
@@ -1518,12 +1531,16 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_cols_fl_kernel(GatBwdArgs<T> a
       cols_edges<T, L, V, DROP, R>(a, ln, ii, ee, ln.g * L, 0, 1, deg, wave_group_max<L>(deg), ac, st);
       cols_quad_reduce<R>(st);
       if constexpr (cols_pairwise<V>()) cols_pair_t<L, W, V>(st, ln, false);
+      if (deg == 0) st.clear();
     } else {
       cols_edges<T, L, V, DROP, R>(a, ln, ii, ee, 0, ln.g, G, deg, (deg + G - 1) / G, ac, st);
       cols_quad_reduce<R>(st);
       cols_group_sum<L, W, V>(st, ln);
     }
     cols_gac(a, ln, st, xc, j, cq, gac);
+    if (deg == 0)
+#pragma unroll
+      for (int v = 0; v < V; ++v) gac[v] = 0.0f;
     if (!(has && (tiny || ln.g == 0))) return;
 #pragma unroll
     for (int v = 0; v < V; ++v) {
@@ -1561,13 +1578,13 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_cols_fl_kernel(GatBwdArgs<T> a
   xc.prefetch(a, ln, j);
   // next round's entries loaded before this round's gathers, as in the forward
   int tb = sg.y + wave * kWave;
-  int ii = tb + ln.lane < sg.z ? a.rowind[tb + ln.lane] : 0;
-  int ee = DROP && tb + ln.lane < sg.z ? a.perm[tb + ln.lane] : 0;
+  int ii = a.rowind[min(tb + ln.lane, sg.z - 1)];
+  int ee = DROP ? a.perm[min(tb + ln.lane, sg.z - 1)] : 0;
   for (; tb < sg.z; tb += kSegRound) {
     const int cnt = min(kWave, sg.z - tb);
     const int tn = tb + kSegRound + ln.lane;
-    const int in = tn < sg.z ? a.rowind[tn] : 0;
-    const int en = DROP && tn < sg.z ? a.perm[tn] : 0;
+    const int in = tn < sg.z ? a.rowind[tn] : ii;
+    const int en = DROP && tn < sg.z ? a.perm[tn] : ee;
     cols_edges<T, L, V, DROP, R>(a, ln, ii, ee, 0, ln.g, G, cnt, (cnt + G - 1) / G, ac, st);
     ii = in;
     ee = en;
@@ -1727,7 +1744,7 @@ struct CmAcc {
 
 // One batch of U slots of a group: slot k's destination row index (and CSR
 // edge id, with dropout) is held by lane src0 + k; slots k >= cnt are unused
-// (their lanes hold index 0, a valid row and edge, read and ignored). c: the
+// (their lanes hold another entry of the column, read and weighted 0). c: the
 // lane's channel chunk; hl: its quad lane (the head whose weights it
 // computes); ac: attn_col of the column for head min(hl, HH - 1).
 #ifndef CIGN_FL_COLS_CM_SHARE
@@ -1859,15 +1876,15 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_cols_cm_kernel(GatBwdArgs<T> a
     const int deg = r.z - r.y;
     const int nb = (deg + U - 1) / U;
     const float ac = a.attn_col[static_cast<int64_t>(j) * HH + hc];
-    int ii = c < U && c < deg ? a.rowind[r.y + c] : 0;
-    int ee = DROP && c < U && c < deg ? a.perm[r.y + c] : 0;
+    int ii = c < U ? list_index(a.rowind, r.y, deg, c) : 0;
+    int ee = DROP && c < U ? list_index(a.perm, r.y, deg, c) : 0;
 #pragma unroll
     for (int h = 0; h < HH; ++h) xr[h] = Four<T>::load(a.x + static_cast<int64_t>(j) * F + h * C + 4 * c);
     for (int bb = 0; bb < nb; ++bb) {
       const int k0 = bb * U;
       const int kn = k0 + U + c;
-      const int in = c < U && kn < deg ? a.rowind[r.y + kn] : 0;
-      const int en = DROP && c < U && kn < deg ? a.perm[r.y + kn] : 0;
+      const int in = c < U && kn < deg ? a.rowind[r.y + kn] : ii;
+      const int en = DROP && c < U && kn < deg ? a.perm[r.y + kn] : ee;
       cm_batch<T, LC, HH, DROP, U>(a, c, hl, ii, ee, g * LC, deg - k0, ac, st);
       ii = in;
       ee = en;
@@ -1880,6 +1897,7 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_cols_cm_kernel(GatBwdArgs<T> a
       const float th = quad_bcast<4, h>(st.t);
       if (c == h) gac = d[h] * a.inv_h - th;
     });
+    if (deg == 0) gac = 0.0f;
 #pragma unroll
     for (int h = 0; h < HH; ++h) {
       float o[4];
@@ -1904,12 +1922,12 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_cols_cm_kernel(GatBwdArgs<T> a
   for (int h = 0; h < HH; ++h) xr[h] = Four<T>::load(a.x + static_cast<int64_t>(j) * F + h * C + 4 * c);
   int tb = sg.y;
   int t0 = tb + gid * U + c;
-  int ii = c < U && t0 < sg.z ? a.rowind[t0] : 0;
-  int ee = DROP && c < U && t0 < sg.z ? a.perm[t0] : 0;
+  int ii = c < U ? a.rowind[min(t0, sg.z - 1)] : 0;
+  int ee = DROP && c < U ? a.perm[min(t0, sg.z - 1)] : 0;
   for (; tb < sg.z; tb += E) {
     const int tn = tb + E + gid * U + c;
-    const int in = c < U && tn < sg.z ? a.rowind[tn] : 0;
-    const int en = DROP && c < U && tn < sg.z ? a.perm[tn] : 0;
+    const int in = c < U && tn < sg.z ? a.rowind[tn] : ii;
+    const int en = DROP && c < U && tn < sg.z ? a.perm[tn] : ee;
     cm_batch<T, LC, HH, DROP, U>(a, c, hl, ii, ee, g * LC, sg.z - (tb + gid * U), ac, st);
     ii = in;
     ee = en;

@@ -210,16 +210,14 @@ struct FwdWave {
 
   __device__ __forceinline__ void load(const GatFwdArgs<T>& a, const Lanes<HP>& L, int eb, int ee, float adst) {
     if (ee <= eb) {
-      // No edges (wave-uniform): nothing is read; eb may equal nnz here.
+      // No edges (wave-uniform): nothing is read (eb may equal nnz here), by
+      // accumulate() neither.
 #pragma unroll
       for (int k = 0; k < N; ++k) {
         t[k] = eb;
         v[k] = false;
-        j[k] = 0;
+        j[k] = -1;
         sc[k] = kNegBig;
-        if constexpr (kPrefetch)
-#pragma unroll
-          for (int c = 0; c < CP; ++c) x0[k][c] = 0.0f;
       }
       return;
     }
@@ -272,6 +270,7 @@ struct FwdWave {
                                              bool normalise, float (&acc)[CP]) const {
 #pragma unroll
     for (int c = 0; c < CP; ++c) acc[c] = 0.0f;
+    if (j[0] < 0) return;  // no edges
     float xv[N][CP];
     if (kPrefetch && cb == 0) {
 #pragma unroll
@@ -694,10 +693,11 @@ template <typename T, int HP, int N>
 __device__ __forceinline__ float bwd_col_wave(const GatBwdArgs<T>& a, const Lanes<HP>& L, int cb0, int ce,
                                               float asrc, int (&i)[N], float (&w)[N]) {
   if (ce <= cb0) {
-    // No edges (wave-uniform): nothing is read; cb0 may equal nnz here.
+    // No edges (wave-uniform): nothing is read (cb0 may equal nnz
+    // here), by the gather neither.
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-      i[k] = 0;
+      i[k] = -1;
       w[k] = 0.0f;
     }
     return 0.0f;
@@ -740,6 +740,11 @@ __device__ __forceinline__ float bwd_col_wave(const GatBwdArgs<T>& a, const Lane
 template <typename T, int CP, int N>
 __device__ __forceinline__ void bwd_col_gather(const GatBwdArgs<T>& a, int cb, const int (&i)[N], const float (&w)[N],
                                                float (&acc)[CP]) {
+  if (i[0] < 0) {  // no edges (wave-uniform)
+#pragma unroll
+    for (int c = 0; c < CP; ++c) acc[c] = 0.0f;
+    return;
+  }
   const int nvalid = min(CP, a.C - cb * CP);
   float gv[N][CP];
 #pragma unroll

@@ -438,3 +438,59 @@ def test_padded_heads_take_pair_layout_schedules(H, C, dtype, monkeypatch):
     test_ext_forward_backward_matches_oracle(H, C, 0.5, dtype, 300, {0: 700, 5: 90}, True, False, monkeypatch)
     with pytest.raises(RuntimeError, match="light_max"):
         test_ext_forward_backward_matches_oracle(4, 16, 0.0, dtype, 300, {0: 700}, True, False, monkeypatch)
+
+
+# Exact and padded shapes of the feature layout (one and several chunks a lane,
+# lane groups of 4, 16, 32 and 64; the channel-major columns at 4 x 16 and 4 x 32)
+# and shapes of the pair layout.
+ISOLATION = [
+    (4, 16, torch.float32), (1, 12, torch.float32), (4, 32, torch.bfloat16), (6, 256, torch.bfloat16),
+    (8, 64, torch.float32), (5, 48, torch.float32), (3, 100, torch.float32), (5, 256, torch.float32),
+    (5, 48, torch.bfloat16), (6, 96, torch.bfloat16), (1, 3, torch.float32), (12, 8, torch.float32),
+]
+
+
+@pytest.mark.parametrize("big", [False, True], ids=["small-graph-kernels", "large-graph-kernels"])
+@pytest.mark.parametrize("agg_mode", [False, True])
+@pytest.mark.parametrize("p", [0.0, 0.3])
+@pytest.mark.parametrize("H,C,dtype", ISOLATION)
+def test_values_that_are_no_numbers_stay_with_their_neighbours(H, C, dtype, p, agg_mode, big, monkeypatch):
+    """NaN and infinities in node 0's features or gradient, node 0 being
+    adjacent to itself only, leave every other node's results as they were,
+    bit for bit: rows and columns whose entries do not fill their lanes, none
+    at all, one segment and several."""
+    from cign_amd.collapsed_gat import ensure_collapsed_gat_loaded
+
+    if big:
+        monkeypatch.setenv("CIGN_GAT_BIG_GRAPH_EDGES", "0")
+    print(f"gat isolation H={H} C={C} dtype={dtype} p={p} agg={agg_mode} big={big}", flush=True)
+    rng = np.random.default_rng(H * C)
+    n = 800
+    # (src, dst) among nodes 2.., every degree up to 70 and hubs of either kind;
+    # node 1 has no edge at all
+    deg = np.concatenate([np.arange(71), rng.integers(0, 12, n - 73)])
+    deg[[100, 200]] = [700, 300]
+    src = np.concatenate([2 + rng.choice(n - 2, size=int(k), replace=False) for k in deg])
+    dst = np.repeat(np.arange(2, n), deg)
+    src, dst = np.concatenate([src, dst, [0]]), np.concatenate([dst, src, [0]])
+    r, c, _ = O.coalesce(src.astype(np.int64), dst.astype(np.int64), n)
+    rowptr, col, row, colptr, perm = _dev_graph(np.stack([r, c]), n)
+    assert not bool(rowptr.diff()[1]) and not bool(colptr.diff()[1]) and int(rowptr.diff().max()) > 512
+    x, ar, ac, b, gy = _inputs(rng, n, H, C, dtype)
+    ext = ensure_collapsed_gat_loaded()
+
+    def results(x, gy):
+        (out, pre, emax, esum, mask), agg = _forward(ext, agg_mode, ar, ac, rowptr, col, 0.2, x, b, p, 7)
+        gx, gar, gac, _ = ext.backward(0.2, p, rowptr, col, colptr, row, perm, emax, esum, mask, x, ar, ac, pre, gy,
+                                       agg)
+        return dict(out=out, pre=pre, edge_max=emax, edge_sum=esum, grad_feat=gx, grad_attn_row=gar,
+                    grad_attn_col=gac)
+
+    want = results(x, gy)
+    assert all(bool(torch.isfinite(v).all()) for v in want.values())
+    for bad in (float("nan"), float("inf"), -float("inf")):
+        for where in ("features", "gradient"):
+            x2, gy2 = x.clone(), gy.clone()
+            (x2 if where == "features" else gy2)[0] = bad
+            for k, v in results(x2, gy2).items():
+                assert torch.equal(v[1:], want[k][1:]), f"{k} with {bad} in node 0's {where}"
