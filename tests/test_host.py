@@ -331,3 +331,19 @@ def test_native_binding_matches_the_library():
             _cign.cign_spmm_partial_bytes(*bad)
     with pytest.raises(TypeError, match="address"):
         _cign.cign_row_schedule_build("x", 3, LIGHT_MAX, SEG_EDGES, out.ctypes.data, out.size)
+
+
+def test_schedule_addresses_are_those_of_the_arrays_it_holds():
+    """Copies, pickles and a replaced header: args() names the object's own
+    arrays, not those of the schedule it was made from."""
+    import copy
+    import pickle
+
+    s = build_row_schedule(torch.tensor([0, 3, 3, 80]), device="cpu")
+    twins = [s, copy.copy(s), copy.deepcopy(s), pickle.loads(pickle.dumps(s))]
+    twins[1].header = s.header.copy()
+    twins[2].header.flags.writeable = False
+    for t in twins:
+        assert t.args() == (t.buf.data_ptr(), t.header.ctypes.data)
+        assert np.array_equal(t.header, s.header)
+    assert len({t.args()[1] for t in twins}) == len(twins)
