@@ -147,8 +147,9 @@ __device__ __forceinline__ void zero(float (&acc)[VPL][W]) {
 
 // First column of the tile's chunk c within its row, from a.c0. Where the row
 // is no whole number of chunks, the last chunk of the row ends at the row's
-// end and repeats columns of the one before it (the same sums, in the same
-// order, stored twice).
+// end and repeats columns of the one before it, which is in the same launch
+// (the same sums, in the same order, stored twice; both have loaded `add` by
+// then).
 template <typename T, int W, int VPL, bool TILED>
 __device__ __forceinline__ int chunk_col(const SpmmArgs<T, W, VPL, TILED>& a, int c) {
   if constexpr (std::is_same<T, f32u>::value || std::is_same<T, bf16u>::value) return min(c * W, a.ld - W - a.c0);
@@ -458,8 +459,12 @@ int launch_all(hipStream_t stream, const Sched& s, const SchedInfo& info, int ld
   constexpr int kChunkBytes = static_cast<int>(sizeof(T)) * W;
   constexpr bool kTiles = W > 1 && std::is_same<T, float>::value;
   constexpr int kTileBytes = 256;
-  for (int ch0 = 0; ch0 < total_ch; ch0 += kMaxCh) {
-    const int nch = min(kMaxCh, total_ch - ch0);
+  for (int ch0 = 0, nch; ch0 < total_ch; ch0 += nch) {
+    nch = min(kMaxCh, total_ch - ch0);
+    // A last chunk that overlaps the one before it (chunk_col) shares its
+    // launch: in a launch of its own it would add `add` again to columns that
+    // are stored, where y is add.
+    if (ld % W != 0 && total_ch - ch0 - nch == 1) --nch;
     const int c0 = ch0 * W;
     // Column tiles of one launch: up to 8, none narrower than 256 bytes (two
     // tiles of 128 at D = 64: 10.9 us against 8.8). Rows of at most 512 bytes

@@ -61,7 +61,8 @@ int64_t cign_spmm_partial_bytes(int32_t n_seg, int32_t d);
 /* y = P x (+ add). One cusparseSpMM of MultiHopCsrPlan::spmm
  * (multihop_csr_pipeline_cuda.cu:264-285) or one torch.sparse.mm of
  * FixedCSRSpMMFunction (model.py:88-106). col/val are the CSR arrays of P
- * whose row pointer the schedule was built from; add may be NULL. */
+ * whose row pointer the schedule was built from; add may be NULL, or y itself
+ * (y += P x). */
 int cign_spmm(void* stream, int32_t dtype, int32_t n_rows, int32_t d, const int32_t* col, const float* val,
               const int32_t* sched, const int32_t* sched_info, const void* x, const void* add, void* y,
               float* partial, int32_t* counters);

@@ -306,3 +306,38 @@ def test_spmm_column_tiles_and_unaligned_rows(dtype, d):
         else:
             assert_within(y.double().cpu().numpy(), ref, _bf16_hop_bound(p, xn, ref, add=add_n), "spmm bf16")
     assert int(parts.sched.counters.abs().sum()) == 0
+
+
+# Rows of one chunk more than a launch takes, whole and in part, and of two.
+@pytest.mark.parametrize("dtype,d", [(torch.float32, d) for d in (33, 1023, 1025, 1026, 1027, 1028, 1029, 2051)] +
+                         [(torch.bfloat16, d) for d in (63, 2049, 2052, 2055, 2057, 4097)])
+def test_spmm_adds_in_place_once(dtype, d):
+    """y = P x + y, the sum written over the term added to it, gives what a
+    separate result gives, bit for bit: light rows of every kind, rows of one
+    and of several segments, no edges."""
+    from cign_amd.graph import HipCsr
+    from cign_amd.schedule import build_row_schedule
+
+    print(f"spmm in place dtype={dtype} d={d}", flush=True)
+    rng = np.random.default_rng(d)
+    n = 700
+    deg = rng.integers(0, 30, n)
+    deg[[3, 650, 0]] = [690, 300, 0]
+    rp = np.concatenate([[0], np.cumsum(deg)])
+    col = np.concatenate([np.sort(rng.choice(n, size=int(k), replace=False)) for k in deg]).astype(np.int64)
+    val = (rng.random(col.size) / np.repeat(np.maximum(deg, 1), deg)).astype(np.float32)
+    crow = torch.from_numpy(rp).cuda()
+    parts = HipCsr(torch.sparse_csr_tensor(crow, torch.from_numpy(col).cuda(), torch.from_numpy(val).cuda(),
+                                           size=(n, n)))
+    parts.sched = build_row_schedule(crow, seg_edges=256)
+    x, add = _rand((n, d), dtype, 3), _rand((n, d), dtype, 4)
+    want = parts.spmm(x, add=add)
+    got = add.clone()
+    assert torch.equal(parts.spmm(x, add=got, out=got), want)
+    ref = O.spmm(rp, col, val.astype(np.float64), x.double().cpu().numpy(), add=add.double().cpu().numpy())
+    if dtype == torch.float32:
+        assert_close(want.cpu().numpy(), ref, name="spmm", **F32_TOL)
+    else:
+        bound = _bf16_hop_bound((rp, col, val.astype(np.float64)), x.double().cpu().numpy(), ref,
+                                add=add.double().cpu().numpy())
+        assert_within(want.double().cpu().numpy(), ref, bound, "spmm bf16")
