@@ -120,9 +120,7 @@ struct SpmmArgs {
   int ld;       // row stride of x / add / y (elements)
   int c0;       // first column of the launch; in the kernel, of the workgroup's tile
   int nch;      // chunks (of W elements) of the launch; in the kernel, of the tile
-  int tch;      // chunks per tile
-  int lgT;      // log2 of the tile slots workgroup ids are dealt over
-  int n_tile;   // tiles (slots past them exit)
+  int lgT;      // log2 of the tiles, over which workgroup ids are dealt
   int width;    // columns of the launch (row stride of `partial`)
   int L;        // lanes per group (power of two, L * VPL >= nch)
   int lgL;      // log2(L)
@@ -213,8 +211,8 @@ __device__ __forceinline__ int wave_max_over_groups(int v, int L) {
 // Gathers `need` (wave-uniform) slots per lane group, at most kSpmmInflight
 // chunks in flight per lane.
 template <typename T, int W, int VPL, bool TILED>
-__device__ __forceinline__ void gather(const SpmmArgs<T, W, VPL, TILED>& a, int jj, float vv, int base, int first, int step,
-                                       int cnt, int need, int gl, float (&acc)[VPL][W]) {
+__device__ __forceinline__ void gather(const SpmmArgs<T, W, VPL, TILED>& a, int jj, float vv, int base, int first,
+                                       int step, int cnt, int need, int gl, float (&acc)[VPL][W]) {
   SpmmBatches<T, W, VPL, TILED> sb{a, jj, vv, base, first, step, cnt, gl, acc};
   for_batches<(kSpmmInflight / VPL > 0 ? kSpmmInflight / VPL : 1)>(need, sb);
 }
@@ -232,14 +230,14 @@ struct AddRow {
 #pragma unroll
     for (int v = 0; v < VPL; ++v) {
       const int c = min(gl + (v << a.lgL), a.nch - 1);
-  raw[v] = Chunk<T, W>::load_raw(base + chunk_col(a, c));
+      raw[v] = Chunk<T, W>::load_raw(base + chunk_col(a, c));
     }
   }
 };
 
 template <typename T, int W, int VPL, bool TILED>
-__device__ __forceinline__ void write_row(const SpmmArgs<T, W, VPL, TILED>& a, int row, int gl, const float (&acc)[VPL][W],
-                                          const AddRow<T, W, VPL, TILED>& ar) {
+__device__ __forceinline__ void write_row(const SpmmArgs<T, W, VPL, TILED>& a, int row, int gl,
+                                          const float (&acc)[VPL][W], const AddRow<T, W, VPL, TILED>& ar) {
 #pragma unroll
   for (int v = 0; v < VPL; ++v) {
     const int c = gl + (v << a.lgL);
@@ -273,9 +271,8 @@ __global__ __launch_bounds__(kSpmmBlock) void spmm_kernel(SpmmArgs<T, W, VPL, TI
   if constexpr (TILED) {
     const int tile = b & ((1 << a.lgT) - 1);
     b >>= a.lgT;
-    if (tile >= a.n_tile) return;
-    a.c0 += tile * a.tch * W;
-    a.nch = min(a.tch, a.nch - tile * a.tch);
+    a.nch >>= a.lgT;
+    a.c0 += tile * a.nch * W;
   }
   float acc[VPL][W];
   zero(acc);
@@ -391,7 +388,7 @@ __global__ __launch_bounds__(kSpmmBlock) void spmm_kernel(SpmmArgs<T, W, VPL, TI
     for (int v = 0; v < kSpmmWaves; ++v) t += red[v][red_at(c)];
     st_agent(part + c, t);
   }
-  if (!arrive_last(a.counters + sg.w, hr.y * a.n_tile, &flag)) return;
+  if (!arrive_last(a.counters + sg.w, hr.y << a.lgT, &flag)) return;
   for (int c = threadIdx.x; c < a.width; c += kSpmmBlock) {
     float t = 0.0f;
     for (int q = 0; q < hr.y; ++q) t += ld_agent(a.partial + static_cast<int64_t>(hr.x + q) * a.width + c);
@@ -415,18 +412,16 @@ struct SchedInfo {
 inline SchedInfo read_info(const int32_t* hdr) { return SchedInfo{hdr, hdr[0], hdr[1], hdr[2]}; }
 
 template <typename T, int W, int VPL, bool TILED>
-int launch_tiles(hipStream_t stream, const Sched& s, const SchedInfo& info, int ld, int c0, int nch, int tch, int lgT,
+int launch_tiles(hipStream_t stream, const Sched& s, const SchedInfo& info, int ld, int c0, int nch, int lgT,
                  const int32_t* col, const float* val, const T* x, const T* add, T* y, float* partial,
                  int32_t* counters) {
   SpmmArgs<T, W, VPL, TILED> a;
   a.ld = ld;
   a.c0 = c0;
   a.nch = nch;
-  a.tch = tch;
   a.lgT = lgT;
-  a.n_tile = (nch + tch - 1) / tch;
   a.width = min(nch * W, ld - c0);
-  const int lanes_needed = (tch + VPL - 1) / VPL;
+  const int lanes_needed = ((nch >> lgT) + VPL - 1) / VPL;
   a.lgL = ilog2(lanes_needed < 1 ? 1 : lanes_needed);
   a.L = 1 << a.lgL;
   a.col = col;
@@ -447,7 +442,8 @@ int launch_tiles(hipStream_t stream, const Sched& s, const SchedInfo& info, int 
   const int64_t blocks = static_cast<int64_t>(s.n_seg + a.mid_blocks + tiny_blocks) << lgT;
   if (blocks == 0) return kOk;
   if (blocks > INT32_MAX) return set_error(kInvalid, "cign_spmm: %lld workgroups", static_cast<long long>(blocks));
-  hipLaunchKernelGGL((spmm_kernel<T, W, VPL, TILED>), dim3(static_cast<unsigned>(blocks)), dim3(kSpmmBlock), 0, stream, a, s);
+  hipLaunchKernelGGL((spmm_kernel<T, W, VPL, TILED>), dim3(static_cast<unsigned>(blocks)), dim3(kSpmmBlock), 0, stream,
+                     a, s);
   return check_launch("cign_spmm");
 }
 
@@ -459,6 +455,7 @@ int launch_all(hipStream_t stream, const Sched& s, const SchedInfo& info, int ld
   constexpr int kChunkBytes = static_cast<int>(sizeof(T)) * W;
   constexpr bool kTiles = W > 1 && std::is_same<T, float>::value;
   constexpr int kTileBytes = 256;
+  constexpr int kLineCh = 128 / kChunkBytes;  // chunks of a 128-byte line (tiled launches)
   for (int ch0 = 0, nch; ch0 < total_ch; ch0 += nch) {
     nch = min(kMaxCh, total_ch - ch0);
     // A last chunk that overlaps the one before it (chunk_col) shares its
@@ -467,22 +464,25 @@ int launch_all(hipStream_t stream, const Sched& s, const SchedInfo& info, int ld
     if (ld % W != 0 && total_ch - ch0 - nch == 1) --nch;
     const int c0 = ch0 * W;
     // Column tiles of one launch: up to 8, none narrower than 256 bytes (two
-    // tiles of 128 at D = 64: 10.9 us against 8.8). Rows of at most 512 bytes
-    // stay whole (D = 128: 13.5 us either way), and so do rows that are no
-    // whole number of 128-byte lines, whose tiles would share lines (D = 200:
-    // 22.8 us whole, 24.0 in two tiles), and bf16 rows, whose lanes unpack
-    // twice the values of a load (D = 512: 29.4 us whole or in two tiles, 46.8
-    // in eight).
+    // tiles of 128 at D = 64: 10.9 us against 8.8), and each a whole number of
+    // 128-byte lines, aligned to them: tiles that share lines fetch those from
+    // two XCDs (D = 200: 22.8 us whole, 24.0 in two tiles; at 24,492 nodes and
+    // 100,000 of 17 entries D = 160 19.9 and 136 us whole, 21.0 and 152 in two
+    // tiles of 320 bytes; 288 31.4 and 247 whole, 34.2 and 297 in four; 640 61.4
+    // and 534 in four, 66.4 and 616 in eight). Rows of at most 512 bytes stay
+    // whole (D = 128: 13.5 us either way), and so do bf16 rows, whose lanes
+    // unpack twice the values of a load (24,492 nodes, D = 512: 29.4 us whole or
+    // in two tiles, 46.8 in eight).
     int lgT = 0;
     if constexpr (kTiles) {
       if (nch * kChunkBytes > 512 && (ld * static_cast<int>(sizeof(T))) % 128 == 0)
-        while (lgT < 3 && (nch >> (lgT + 1)) * kChunkBytes >= kTileBytes) ++lgT;
+        while (lgT < 3 && (nch >> (lgT + 1)) * kChunkBytes >= kTileBytes && (nch >> lgT) % (2 * kLineCh) == 0) ++lgT;
     }
-    const int tch = (nch + (1 << lgT) - 1) >> lgT;
+    const int tch = nch >> lgT;
     const int vpl = tch <= (lgT == 0 ? kWave : 16) ? 1 : tch <= 2 * kWave ? 2 : 4;
     int rc = kOk;
 #define CIGN_SPMM_LAUNCH(VPL, TILED)                                                                             \
-  rc = launch_tiles<T, W, VPL, TILED>(stream, s, info, ld, c0, nch, tch, lgT, col, val, x, add, y, partial, counters)
+  rc = launch_tiles<T, W, VPL, TILED>(stream, s, info, ld, c0, nch, lgT, col, val, x, add, y, partial, counters)
     if (lgT == 0) {
       if (vpl == 1) CIGN_SPMM_LAUNCH(1, false);
       else if (vpl == 2) CIGN_SPMM_LAUNCH(2, false);

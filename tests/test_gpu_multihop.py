@@ -341,3 +341,10 @@ def test_spmm_adds_in_place_once(dtype, d):
         bound = _bf16_hop_bound((rp, col, val.astype(np.float64)), x.double().cpu().numpy(), ref,
                                 add=add.double().cpu().numpy())
         assert_within(want.double().cpu().numpy(), ref, bound, "spmm bf16")
+
+
+@pytest.mark.parametrize("d", [224, 288, 320, 352, 448, 480, 640, 832, 960, 1184])
+def test_spmm_tiles_of_whole_lines(d):
+    """fp32 widths whose tiles are fewer than eight because they are whole
+    128-byte lines (several chunks a lane), or that stay whole."""
+    test_spmm_column_tiles_and_unaligned_rows(torch.float32, d)
