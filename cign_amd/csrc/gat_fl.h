@@ -230,13 +230,13 @@ __device__ __forceinline__ void store_values(T* p, const float (&v)[W]) {
 }
 
 // Index of entry `slot` of the list at p (deg entries from `first`), or for a
-// lane past its end of the list's first entry: the batches read whatever row a
+// lane past its end of the list's last entry: the batches read whatever row a
 // lane's index names and give a slot past the end weight 0, so that row has to
 // be one the list's owner reads anyway. (Index 0 there carried a NaN or an
 // infinity of node 0, 0 times it, into nearly every row.) An empty list reads
 // nothing and has index 0; its owner drops what its slots added.
 __device__ __forceinline__ int list_index(const int32_t* p, int first, int deg, int slot) {
-  return deg > 0 ? p[first + (slot < deg ? slot : 0)] : 0;
+  return deg > 0 ? p[first + min(slot, deg - 1)] : 0;
 }
 
 // Largest value of v over the groups of a wavefront (lane bits >= log2 L).
