@@ -1637,21 +1637,29 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_cols_fl_kernel(GatBwdArgs<T> a
   }
   if (single) return;
   if (!arrive_last(a.col_counters + sg.w, hr.y, &flag)) return;
-  if (threadIdx.x < a.H) {
-    float v = 0.0f;
-    for (int z = 0; z < hr.y; ++z) v += ld_agent(a.part_col + static_cast<int64_t>(hr.x + z) * stride + F + threadIdx.x);
-    a.grad_attn_col[static_cast<int64_t>(j) * a.H + threadIdx.x] = v;
-    gred[0][threadIdx.x] = v;
-  }
-  __syncthreads();
-  for (int k = threadIdx.x; k < F; k += kBlock) {
+  const auto total = [&](int k) {
     float v = 0.0f;
     for (int z = 0; z < hr.y; ++z) v += ld_agent(a.part_col + static_cast<int64_t>(hr.x + z) * stride + k);
-    if (proj) {
-      if constexpr (kGatProj<T>) store_proj1(a, j, k / a.C, k, v * a.inv_h, gred[0][k / a.C]);
-    } else {
-      a.grad_feat[static_cast<int64_t>(j) * F + k] = from_f32<GatOut<T>>(v * a.inv_h);
+    return v;
+  };
+  // (one loop where nothing waits for grad_attn_col: in two the hub columns'
+  // merges were the launch's tail, 10.9 us against 10.5 at 24,492 x 4 x 16)
+  if (!proj) {
+    for (int k = threadIdx.x; k < stride; k += kBlock) {
+      const float v = total(k);
+      if (k < F) a.grad_feat[static_cast<int64_t>(j) * F + k] = from_f32<GatOut<T>>(v * a.inv_h);
+      else a.grad_attn_col[static_cast<int64_t>(j) * a.H + (k - F)] = v;
     }
+    return;
+  }
+  if constexpr (kGatProj<T>) {  // grad_attn_col first: every element of its head needs it
+    if (threadIdx.x < a.H) {
+      const float v = total(F + threadIdx.x);
+      a.grad_attn_col[static_cast<int64_t>(j) * a.H + threadIdx.x] = v;
+      gred[0][threadIdx.x] = v;
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < F; k += kBlock) store_proj1(a, j, k / a.C, k, total(k) * a.inv_h, gred[0][k / a.C]);
   }
 }
 
