@@ -1487,12 +1487,21 @@ using GatProj = std::conditional_t<std::is_same_v<T, bf16x>, bf16, GatOut<T>>;
 template <typename T>
 constexpr bool kGatProj = std::is_same_v<T, float> || std::is_same_v<T, bf16x>;
 
+// grad_feat plus the logits' terms, each rounded as in the two passes that this
+// replaces (grad_feat, the terms' sum, their sum), so that it is the same
+// number: contracted with the product grad_feat comes from, it fell on the other
+// side of a bf16 rounding now and then.
+__device__ __forceinline__ float proj_grad(float grad_feat, float gac, float as, float gar, float ad) {
+#pragma clang fp contract(off)
+  return grad_feat + fmaf(gac, as, gar * ad);
+}
+
 // Element k = h C + c of column j's projection gradient from its grad_feat
 // value v and the column's grad_attn_col of head h.
 template <typename T>
 __device__ __forceinline__ void store_proj1(const GatBwdArgs<T>& a, int j, int h, int k, float v, float gac) {
   const float gar = a.grad_attn_row[static_cast<int64_t>(j) * a.H + h];
-  const float g = v + (gac * a.att_src[k] + gar * a.att_dst[k]);
+  const float g = proj_grad(v, gac, a.att_src[k], gar, a.att_dst[k]);
   reinterpret_cast<GatProj<T>*>(a.grad_feat)[static_cast<int64_t>(j) * a.H * a.C + k] = from_f32<GatProj<T>>(g);
 }
 
@@ -1573,7 +1582,7 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_cols_fl_kernel(GatBwdArgs<T> a
           load_f32<W>(a.att_src + ln.off[v], as);
           load_f32<W>(a.att_dst + ln.off[v], ad);
 #pragma unroll
-          for (int w = 0; w < W; ++w) o[w] += gac[v] * as[w] + gar * ad[w];
+          for (int w = 0; w < W; ++w) o[w] = proj_grad(o[w], gac[v], as[w], gar, ad[w]);
           store_values<GatProj<T>, W>(
               reinterpret_cast<GatProj<T>*>(a.grad_feat) + static_cast<int64_t>(j) * F + ln.off[v], o);
         }

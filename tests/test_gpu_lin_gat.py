@@ -385,6 +385,45 @@ def test_gat_backward_with_logits(H, C, hold, p):
     assert torch.equal(vecs[0], vecs[1])
 
 
+@pytest.mark.parametrize("H,C,hold", [(6, 256, True), (6, 256, False), (4, 64, True), (8, 256, True), (5, 48, False),
+                                      (7, 256, False)])
+def test_projection_gradient_is_that_of_the_two_passes(H, C, hold):
+    """cign_gat_bwd_logits gives the bits of cign_gat_bwd followed by
+    cign_attn_logits_bwd_acc, in float32 and, held, rounded to bf16; columns
+    without entries, light, of one segment and of several."""
+    from cign_amd import _lib
+    from cign_amd.collapsed_gat import ensure_collapsed_gat_loaded
+    from oracle import cign_oracle as O
+
+    print(f"projection gradient H={H} C={C} hold={hold}", flush=True)
+    lib = _lib.load_library()
+    rng = np.random.default_rng(H + C)
+    n = 1500
+    deg = np.concatenate([[0, 1400, 300, 65], rng.integers(0, 60, n - 4)])  # of the columns
+    src = np.repeat(np.arange(n), deg)
+    dst = np.concatenate([rng.choice(n, size=int(k), replace=False) for k in deg])
+    r, c, _ = O.coalesce(src.astype(np.int64), dst.astype(np.int64), n)
+    rowptr, col, row, colptr, perm = _dev_graph(np.stack([r, c]), n)
+    assert colptr.diff().tolist()[:4] == [0, 1400, 300, 65]
+    dt = torch.bfloat16 if hold else torch.float32
+    f = lambda *s: torch.from_numpy(rng.standard_normal(s).astype(np.float32)).cuda()
+    x, ar, ac, b, gy, s, d = f(n, H, C).to(dt), f(n, H), f(n, H), f(C), f(n, C), f(H, C), f(H, C)
+    ext = ensure_collapsed_gat_loaded()
+    (_, pre, emax, esum, mask), agg = ext.forward_agg(ar, ac, rowptr, col, 0.2, x, b, 0.0, 0, True, f32_out=hold)
+    args = (0.2, 0.0, rowptr, col, colptr, row, perm, emax, esum, mask, x, ar, ac, pre, gy, agg)
+    gx, g_row, g_col, _ = ext.backward(*args, f32_out=hold)
+    proj, p_row, p_col, _ = ext.backward(*args, f32_out=hold, logits=(s, d))
+    assert torch.equal(p_row, g_row) and torch.equal(p_col, g_col)
+    want = torch.empty((n, H, C), dtype=dt, device="cuda")
+    ws_bytes = int(lib.cign_colsum_workspace_bytes(n, H * C, 2))
+    ws, vecs = _lib.workspace(ws_bytes, x.device), torch.empty((2, H, C), device="cuda")
+    code = 1 if hold else 0
+    lib.call("cign_attn_logits_bwd_acc", _lib.stream_ptr(x.device), n, H, C, code, code, g_col.data_ptr(),
+             g_row.data_ptr(), x.data_ptr(), s.data_ptr(), d.data_ptr(), gx.data_ptr(), want.data_ptr(),
+             vecs[0].data_ptr(), vecs[1].data_ptr(), ws.data_ptr(), ws_bytes)
+    assert torch.equal(proj, want)
+
+
 def test_gat_backward_with_logits_refuses_other_kernels():
     from cign_amd import _lib
 
