@@ -109,8 +109,18 @@ _LIB_ERROR: BaseException | None = None
 _GPU_SEEN = False
 
 
-# Entry points whose Python callers pass ctypes references (host outputs).
-_BY_REFERENCE = ("cign_row_schedule_size", "cign_gat_schedule_params")
+def _native_first(native, general):
+    """``native``, and for arguments that only ctypes converts (byref, arrays,
+    c_void_p and other ctypes values, bytes) ``general``: _cign.so raises
+    TypeError before it calls the library."""
+
+    def call(*args):
+        try:
+            return native(*args)
+        except TypeError:
+            return general(*args)
+
+    return call
 
 
 class _Lib:
@@ -121,7 +131,7 @@ class _Lib:
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
-            self._fn[name] = fn if name in _BY_REFERENCE else getattr(native, name, fn)
+            self._fn[name] = _native_first(getattr(native, name), fn) if hasattr(native, name) else fn
             sizes = name.endswith(("_bytes", "_floats", "_ok"))
             setattr(self, name, self._fn[name] if sizes else fn)
 

@@ -347,3 +347,23 @@ def test_schedule_addresses_are_those_of_the_arrays_it_holds():
         assert t.args() == (t.buf.data_ptr(), t.header.ctypes.data)
         assert np.array_equal(t.header, s.header)
     assert len({t.args()[1] for t in twins}) == len(twins)
+
+
+def test_calls_take_ctypes_arguments():
+    """call() and the size functions take what ctypes converts beside Python
+    numbers (references, arrays, ctypes values), and refuse the rest as it does."""
+    C = ctypes
+    lib = _lib.load_library(require_gpu=False)
+    rowptr = (C.c_int64 * 4)(0, 3, 3, 80)
+    n = [C.c_int32() for _ in range(3)]
+    total = C.c_int64()
+    lib.call("cign_row_schedule_size", rowptr, C.c_int32(3), LIGHT_MAX, SEG_EDGES, *map(C.byref, n), C.byref(total))
+    out = (C.c_int32 * total.value)()
+    lib.call("cign_row_schedule_build", C.byref(rowptr), 3, C.c_int32(LIGHT_MAX), SEG_EDGES, out, total)
+    s = build_row_schedule(torch.tensor([0, 3, 3, 80]), device="cpu")
+    assert list(out) == s.buf.tolist() and [v.value for v in n] == [s.n_light, s.n_seg, s.n_hrow]
+    assert lib.cign_spmm_partial_bytes(C.c_int32(5), 64) == lib.cign_spmm_partial_bytes(5, 64)
+    with pytest.raises(RuntimeError, match="buffer size mismatch"):
+        lib.call("cign_row_schedule_build", rowptr, 3, LIGHT_MAX, SEG_EDGES, out, total.value - 1)
+    with pytest.raises(C.ArgumentError):
+        lib.call("cign_row_schedule_build", 1.5, 3, LIGHT_MAX, SEG_EDGES, out, total.value)
