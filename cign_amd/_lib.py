@@ -209,8 +209,8 @@ def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
 
 
-def stream_ptr(device: torch.device | None = None) -> int:
-    if device is None or device.type != "cuda" or device.index is None:
+def stream_ptr(device: torch.device | int | str | None = None) -> int:
+    if not isinstance(device, torch.device) or device.type != "cuda" or device.index is None:
         return torch.cuda.current_stream(device).cuda_stream
     # the handle alone: torch.cuda.current_stream builds a Stream object (3 us)
     return torch._C._cuda_getCurrentRawStream(device.index)

@@ -69,3 +69,13 @@ def test_graph_replays_match_eager(dtype, p):
         torch.cuda.synchronize()
         for i, (a, e) in enumerate(zip(static, eager)):
             assert torch.equal(a, e), f"replay {r}: output {i} differs from the eager result"
+
+
+def test_stream_of_a_device_in_any_form():
+    from cign_amd import _lib
+
+    side = torch.cuda.Stream()
+    for stream in (torch.cuda.current_stream(), side):
+        with torch.cuda.stream(stream):
+            for dev in (None, 0, "cuda:0", "cuda", torch.device("cuda"), torch.device("cuda:0")):
+                assert _lib.stream_ptr(dev) == stream.cuda_stream
