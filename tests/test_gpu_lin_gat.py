@@ -349,12 +349,14 @@ def test_gat_backward_with_logits(H, C, hold, p):
     rng = np.random.default_rng(H * C + hold)
     n = 1500
     ei = _graph(rng, n, {2: 1400, 7: 300})
-    out = np.stack([np.full(1400, 11), rng.permutation(n)[:1400]])  # a source of many segments
+    # sources of several segments and, 17, of one
+    out = np.stack([np.repeat([11, 17], [1400, 300]), np.concatenate([rng.permutation(n)[:k] for k in (1400, 300)])])
     from oracle import cign_oracle as O
     r, c, _ = O.coalesce(np.concatenate([ei[0], out[0]]), np.concatenate([ei[1], out[1]]), n)
     ei = np.stack([r, c])
     rowptr, col, row, colptr, perm = _dev_graph(ei, n)
-    assert int(colptr.diff().max()) > 1024
+    deg = colptr.diff()
+    assert int(deg.max()) > 1024 and bool(((deg > 64) & (deg <= 512)).any())
     assert lib.cign_gat_bwd_logits_ok(code, H, C, col.numel()) == 1
     dt = torch.bfloat16 if hold else torch.float32
     f = lambda *s: torch.from_numpy(rng.standard_normal(s).astype(np.float32)).cuda()
