@@ -324,8 +324,13 @@ __global__ __launch_bounds__(kSpmmBlock) void spmm_kernel(SpmmArgs<T, W, VPL, TI
       gather(a, jj, vv, g << a.lgL, 0, 1, deg, wave_max_over_groups(deg, a.L), gl, acc);
     }
     // A group's slots past its row's end reload an edge of that row; a row with
-    // no edge has read another row's.
-    if (deg == 0) zero(acc);
+    // no edge has read another row's. (Rows of several chunks a lane have whole
+    // wavefronts, so no light row comes here but in tiled launches; the sums'
+    // second life costs bf16 rows 2 registers and with them a sixth wavefront per
+    // SIMD: D = 640 39.0 us without, 42.8 with.)
+    if constexpr (TILED || VPL == 1) {
+      if (deg == 0) zero(acc);
+    }
     if (has) write_row(a, r.x, gl, acc, ar);
     return;
   }
@@ -422,7 +427,10 @@ int launch_tiles(hipStream_t stream, const Sched& s, const SchedInfo& info, int 
   a.lgT = lgT;
   a.width = min(nch * W, ld - c0);
   const int lanes_needed = ((nch >> lgT) + VPL - 1) / VPL;
-  a.lgL = ilog2(lanes_needed < 1 ? 1 : lanes_needed);
+  // Unaligned rows of three or four chunks (bf16) take a group of eight lanes:
+  // in a smaller one no light row shares its wavefront (n_mid below).
+  constexpr int kMinLgL = std::is_same<T, f32u>::value || std::is_same<T, bf16u>::value ? 3 : 0;
+  a.lgL = max(kMinLgL, ilog2(lanes_needed < 1 ? 1 : lanes_needed));
   a.L = 1 << a.lgL;
   a.col = col;
   a.val = val;
@@ -509,7 +517,11 @@ int spmm_dispatch(hipStream_t stream, const Sched& s, const SchedInfo& info, int
   if (d % kVec == 0 && aligned) {
     return launch_all<T, kVec>(stream, s, info, d, col, val, xt, at, yt, partial, counters);
   }
-  if (d >= kVec) {
+  // One value a lane up to 16 columns: a lane group of those widths has eight or
+  // sixteen lanes either way, and chunks leave most of them idle (one value a
+  // lane / chunks, us at 24,492 and 100,000 nodes: fp32 D = 5 6.3 and 30 / 9.6
+  // and 39, 15 7.0 and 32 / 9.4 and 44, 17 8.9 and 45 / 7.2 and 41).
+  if (d > 16) {
     using U = typename std::conditional<sizeof(T) == 4, f32u, bf16u>::type;
     return launch_all<U, kVec>(stream, s, info, d, col, val, reinterpret_cast<const U*>(xt),
                                reinterpret_cast<const U*>(at), reinterpret_cast<U*>(yt), partial, counters);

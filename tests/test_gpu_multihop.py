@@ -348,3 +348,30 @@ def test_spmm_tiles_of_whole_lines(d):
     """fp32 widths whose tiles are fewer than eight because they are whole
     128-byte lines (several chunks a lane), or that stay whole."""
     test_spmm_column_tiles_and_unaligned_rows(torch.float32, d)
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.float32, d) for d in (5, 7, 9, 15, 16, 17, 33)] +
+                         [(torch.bfloat16, d) for d in (9, 16, 17, 24, 31, 32, 33)])
+def test_spmm_narrow_unaligned_rows(dtype, d):
+    """Rows that are not 16-byte aligned, one value a lane up to 16 columns and
+    in chunks from 17 on: a light row belongs to one lane group of at least
+    eight lanes and is summed in edge order, the float32 sum in that order bit
+    for bit (weights of one, so a product rounds nothing)."""
+    from cign_amd.graph import HipCsr
+
+    print(f"spmm narrow dtype={dtype} d={d}", flush=True)
+    rng = np.random.default_rng(d)
+    n = 900
+    deg = rng.integers(0, 9, n)
+    rp = np.concatenate([[0], np.cumsum(deg)])
+    col = np.concatenate([np.sort(rng.choice(n, size=int(k), replace=False)) for k in deg]).astype(np.int64)
+    parts = HipCsr(torch.sparse_csr_tensor(torch.from_numpy(rp).cuda(), torch.from_numpy(col).cuda(),
+                                           torch.ones(col.size, device="cuda"), size=(n, n)))
+    x = _rand((n * d + 1,), dtype, 3)[1:].view(n, d)
+    y = parts.spmm(x)
+    xn = x.float().cpu().numpy()
+    want = np.zeros((n, d), np.float32)
+    for i in range(n):
+        for j in col[rp[i]:rp[i + 1]]:
+            want[i] = want[i] + xn[j]
+    assert torch.equal(y.cpu(), torch.from_numpy(want).to(dtype))
