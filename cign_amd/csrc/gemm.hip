@@ -1289,32 +1289,51 @@ __device__ __forceinline__ bool wg_tile_chunk(int tiles, int chunks, bool xcd, i
 inline unsigned wg_grid(int tiles, int chunks, bool xcd) {
   return static_cast<unsigned>(tiles * (xcd ? (chunks + 7) / 8 * 8 : chunks));
 }
-// Row chunks of those kernels: 512 workgroups over the tiles at most, and
-// chunks of at least 128 rows (4 k-steps of kWgM: fewer spend longer filling
-// the pipeline and on the partials than the extra workgroups save), or 64
-// where even so fewer than 64 workgroups run. With bf16 operands 256 rows
-// where that already gives each CU a workgroup. The launches are latency
-// bound while the chip is short of workgroups; fixed 256-row chunks against
-// this rule, with the partials' sum, us:
-//   grad_W fp32  2,000 x 256 x 64: 30.4, 13.9    5,000 x 256 x 128: 27.4, 19.7
-//                1,200 x 512 x 300: 30.4, 22.8   11,003 x 480 x 96: 38.0, 34.9
-//                24,492 x 192 x 192: 51.7, 43.8
-//   grad_W bf16  2,000 x 256 x 64: 17.4, 10.8    11,003 x 96 x 576: 24.7, 22.0
-//   pack projection's backward, D x K, fp32
-//                2,000 x 64 x 2: 62.0, 41.8      24,492 x 64 x 3: 112.6, 100.8
-//   the same in bf16 at 11,003 x 128 x 3 (258 workgroups of 256 rows): 90.4
-//   with 256-row chunks, 98.3 with 128: twice the partials for one more round
-//   of a chip that has one already; so bf16 keeps 256 there.
-// Chunks of 32 rows were slower than 64 from 64 workgroups on (5,000 x 256 x
-// 128: 21.3 against 17.3 with 64). With `xcd` a multiple of 8 chunks (one per
-// XCD each round) once there are at least 8.
-inline int64_t wg_chunk_count(int64_t M, int64_t tiles, bool xcd) {
-  const auto by = [&](int64_t rows) { return (M + rows - 1) / rows; };
-  int64_t rows = 128;
-  if (xcd && tiles * by(256) >= 256) rows = 256;
-  else if (tiles * by(128) < 64) rows = 64;
-  const int64_t c = std::max<int64_t>(1, std::min<int64_t>(by(rows), std::max<int64_t>(1, 512 / tiles)));
-  return xcd && c >= 8 ? (c + 7) / 8 * 8 : c;
+// Kernels whose row chunks wg_chunk_count counts.
+enum WgKind {
+  kWgF32,     // 128 x 128 tiles, fp32 operands
+  kWgBF16,    // the same, bf16 operands
+  kWgNarrow,  // wgrad_narrow_kernel's 64-wide k tiles
+};
+
+// Row chunks of a gradient of N x K values in `tiles` tiles: 512 workgroups at
+// most, then, but for kWgF32, rounded up to a multiple of 8 chunks (one per XCD
+// each round) once there are 8 (24 tiles: 21 chunks, so 24 and 576 workgroups).
+// A chunk is 128 rows (4 k-steps of kWgM), or 64 where even so fewer than 64
+// workgroups run: while the chip is short of workgroups a launch takes as long
+// as its chunk's chain of k-steps. It is 256 rows where shorter chunks cost more
+// than they save:
+// - one round of 256 workgroups takes all chunks of 256 rows but not those of
+//   128, and the chain is short beside a chunk's partials: whole 128 x 128 tiles,
+//   the narrow kernel, and outputs of at least 65,536 values, whose sum walks the
+//   partials in a chain of its own (colsum_wide_kernel).
+// - kWgBF16 and a smaller output: 256 rows fill the round.
+// - kWgBF16 and an output of 65,536 values: more than 5 MB of partials in more
+//   than 4 chunks (the bf16 chain is short in any case).
+// us with the partials' sum, chunks of 64 / 128 / 256 rows, * the choice:
+//   fp32  2,000 x 256 x 64  19.4* 24.0 35.8     5,000 x 256 x 128  24.6 26.5* 33.5
+//         11,003 x 480 x 96  41.3 43.1* 47.4    24,492 x 256 x 128 41.5 43.1 41.0*
+//         11,003 x 256 x 256 60.1 58.4 48.3*    5,000 x 768 x 256  48.0 48.2 42.5*
+//         1,200 x 1536 x 256 34.9 31.8* 36.8    24,492 x 192 x 192 - 43.8* 51.7
+//   bf16  2,000 x 256 x 64  16.3* 17.6 22.9     11,003 x 96 x 576  29.0 28.9* 31.4
+//         2,000 x 256 x 256 24.1 20.0* 20.6     5,000 x 256 x 256  43.1 31.6 26.1*
+//         1,200 x 1536 x 256 29.6 28.3 23.5*    2,000 x 768 x 256  32.2 26.1 22.6*
+//   narrow 2,000 x 64 x 64  13.4* 14.5 16.7     5,000 x 64 x 300   19.3 17.3* 18.7
+//         11,003 x 64 x 300 22.9 23.1 20.9*     60,000 x 64 x 64   26.4 26.5 24.7*
+inline int64_t wg_chunk_count(int64_t M, int64_t tiles, WgKind kind, int64_t N, int64_t K) {
+  const auto count = [&](int64_t rows) {
+    const int64_t c = std::max<int64_t>(1, std::min((M + rows - 1) / rows, std::max<int64_t>(1, 512 / tiles)));
+    return kind != kWgF32 && c >= 8 ? (c + 7) / 8 * 8 : c;
+  };
+  const auto groups = [&](int64_t rows) { return tiles * ((M + rows - 1) / rows); };
+  const bool wide = N * K >= 65536;
+  const auto fits = [&](int64_t rows) {
+    if (kind == kWgBF16) return wide ? count(rows) <= 4 || count(rows) * N * K <= 1250000 : groups(256) < 256;
+    return !(wide || kind == kWgNarrow || (N % kWgT == 0 && K % kWgT == 0)) ||
+           groups(rows) <= 256 || groups(256) > 256;
+  };
+  if (groups(128) < 64 && fits(64)) return count(64);
+  return count(fits(128) ? 128 : 256);
 }
 
 // gy: fp32, or bf16 storage (TG = bf16h: a gradient the caller has rounded to
@@ -3112,7 +3131,7 @@ inline BwdWs bwd_ws(int64_t M, int N, int K, bool bias, bool xcd) {
     const int64_t ntk = (K + kWnK - 1) / kWnK;
     // (about 512: fewer workgroups left the chip short, more spent longer
     // on the chunk partials and their sums than they saved, at the c2 lin)
-    int64_t wgc = wg_chunk_count(M, ntk, true);
+    int64_t wgc = wg_chunk_count(M, ntk, kWgNarrow, N, K);
     L.wg_chunk = std::max<int64_t>(kWnChunkRows,
                                    ((M + wgc - 1) / wgc + kWnChunkRows - 1) / kWnChunkRows * kWnChunkRows);
     wgc = M > 0 ? (M + L.wg_chunk - 1) / L.wg_chunk : 1;
@@ -3123,7 +3142,7 @@ inline BwdWs bwd_ws(int64_t M, int N, int K, bool bias, bool xcd) {
     return L;
   }
   const int64_t tiles = static_cast<int64_t>((N + kWgT - 1) / kWgT) * ((K + kWgT - 1) / kWgT);
-  int64_t wgc = wg_chunk_count(M, tiles, xcd);
+  int64_t wgc = wg_chunk_count(M, tiles, xcd ? kWgBF16 : kWgF32, N, K);
   L.wg_chunk = std::max<int64_t>(kWgM, ((M + wgc - 1) / wgc + kWgM - 1) / kWgM * kWgM);
   wgc = M > 0 ? (M + L.wg_chunk - 1) / L.wg_chunk : 1;
   L.wg_chunks = static_cast<int>(wgc);
@@ -3151,7 +3170,7 @@ inline PpWs pp_ws(int64_t M, int D, int K, bool xcd) {
   auto al = [](int64_t v) { return (v + 255) & ~int64_t(255); };
   const int64_t kw = 2LL * K * D;
   const int64_t tiles = static_cast<int64_t>((D + kWgT - 1) / kWgT) * pp_ntk(D, K);
-  int64_t wgc = wg_chunk_count(M, tiles, xcd);
+  int64_t wgc = wg_chunk_count(M, tiles, xcd ? kWgBF16 : kWgF32, D, kw);
   L.wg_chunk = std::max<int64_t>(kWgM, ((M + wgc - 1) / wgc + kWgM - 1) / kWgM * kWgM);
   L.wg_chunks = static_cast<int>(M > 0 ? (M + L.wg_chunk - 1) / L.wg_chunk : 1);
   int64_t bc = std::max<int64_t>(1, std::min<int64_t>(1024, (M + 63) / 64));
@@ -3314,7 +3333,7 @@ struct WlWs {
 inline WlWs wl_ws(int64_t M, int N, int K) {
   WlWs L;
   L.ntk = (K + kWnK - 1) / kWnK;
-  int64_t wgc = wg_chunk_count(M, L.ntk, true);
+  int64_t wgc = wg_chunk_count(M, L.ntk, kWgNarrow, N, K);
   L.chunk = std::max<int64_t>(kWnChunkRows, ((M + wgc - 1) / wgc + kWnChunkRows - 1) / kWnChunkRows * kWnChunkRows);
   wgc = M > 0 ? (M + L.chunk - 1) / L.chunk : 1;
   L.chunks = static_cast<int>(wgc);

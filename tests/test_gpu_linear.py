@@ -88,8 +88,13 @@ def _check_amp_backward(gy, x, w, gx, gw, gb):
 @pytest.mark.parametrize("M,N,K", [
     (1, 256, 64), (63, 256, 64), (65, 256, 64), (2000, 256, 64),  # 64-row chunks
     (3968, 256, 64), (3969, 256, 64),  # 2 tiles: 64 rows up to 31 chunks of 128, then 128
-    (1792, 512, 1024), (1793, 512, 1024),  # 32 tiles, bf16: 256 rows once 8 such chunks
+    (1792, 512, 1024), (1793, 512, 1024),  # 32 tiles: 7 and 8 chunks of 256 rows
     (511, 64, 256), (1920, 64, 256), (1921, 64, 256),  # the narrow kernel, 4 tiles
+    (512, 512, 1024), (513, 512, 1024),  # bf16: 4 chunks of 128 rows, then 256
+    (2048, 256, 256), (2049, 256, 256),  # bf16: 128 rows up to 5 MB of partials, then 256
+    (8192, 256, 256), (8193, 256, 256),  # fp32, 4 tiles: 128 rows for one round of workgroups, then 256
+    (16384, 256, 256), (16385, 256, 256),  # and 128 again once 256 rows are more than one round
+    (8192, 64, 256), (8193, 64, 256), (16385, 64, 256),  # the same, the narrow kernel
 ])
 @pytest.mark.parametrize("amp", [False, True])
 def test_weight_gradient_row_chunks(M, N, K, amp):
