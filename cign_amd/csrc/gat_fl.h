@@ -111,10 +111,17 @@ constexpr int kFwdUBig = CIGN_FL_FWD_U_BIG;
 // keep 16.
 constexpr int kFwdUNarrowF32 = 8;
 constexpr int kRowsU = CIGN_FL_ROWS_U;
-// Rows of 8-value (bf16) chunks: half of it. 6 x 256 (three chunks a lane),
-// 211K edges: the rows pass 101 us with 4 slots (233 VGPRs), 93 with 2; 4-value
-// chunks keep the larger batch (5 x 96: 38 us against 48).
+// Rows of 8-value (bf16) chunks: half of it, but the whole in rows of several
+// chunks a lane where there are few rows or they are the widest. The larger
+// batch has fewer rounds and the registers of two wavefronts per SIMD; from
+// about 16K rows on the wavefronts the smaller one has room for are worth more.
+// GAT backward, us, 16 slots / 8: 6 x 256 at 2,000 nodes 52.5 / 55.1, 11,003
+// 105.6 / 116.7, 24,492 172.4 / 159.7; 4 x 256 40.0 / 40.7, 80.1 / 86.8, 120.7 /
+// 117.8 (with dropout 145 / 127); 8 x 256 59.0 / 63.8, 117.8 / 129.4, 202 / 208;
+// one chunk a lane, 4 x 32 127.5 / 127.6 at 60,000, 601 / 468 at 240,000. 4-value
+// chunks keep the larger batch (5 x 96: the rows pass 38 us against 48).
 constexpr int kRowsUWide = CIGN_FL_ROWS_U / 2;
+constexpr int kRowsUWideRows = 16384;
 constexpr int kColsU = CIGN_FL_COLS_U;
 // Batch cap of the shared-weight columns batches (large graphs): 4 slots
 // measured 3.54 ms at 62.4M edges against 3.90 ms for 8 and 5.55 ms for 16.
@@ -871,12 +878,12 @@ struct RowBatches {
   }
 };
 
-template <typename T, int L, int V, bool DROP>
+template <typename T, int L, int V, bool DROP, int UM>
 __device__ __forceinline__ void rows_edges(const GatBwdArgs<T>& a, const FlLane<L, V>& ln, int jj, int base,
                                            int first, int step, int cnt, int need, int ebase, const RowHead<V>& rh,
                                            RowAcc<FlGeom<T>::W, V>& st) {
   RowBatches<T, L, V, DROP> rb{a, ln, jj, base, first, step, cnt, ebase, rh, st};
-  for_batches<batch_cap(FlGeom<T>::W == 8 ? kRowsUWide : kRowsU, V)>(need, rb);
+  for_batches<batch_cap(UM, V)>(need, rb);
 }
 
 template <int L, int W, int V>
@@ -966,7 +973,7 @@ __device__ __forceinline__ void rows_emit(const GatBwdArgs<T>& a, const FlLane<L
   if (ln.qv[0] && ln.hq[0] == 0) store_f32<W>(a.grad_pre + static_cast<int64_t>(row) * a.gp_stride + ln.cw * W, gp);
 }
 
-template <typename T, int L, int V, bool DROP>
+template <typename T, int L, int V, bool DROP, int UM>
 __global__ __launch_bounds__(kBlock) void gat_bwd_rows_fl_kernel(GatBwdArgs<T> a, Sched s, int n_mid, int mid_blocks,
                                                                  int lgcq) {
   constexpr int W = FlGeom<T>::W;
@@ -1003,9 +1010,9 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_rows_fl_kernel(GatBwdArgs<T> a
     const RowHead<V> rh = row_head(a, row, ln);
     grad_pre_chunk(a, row, ln.cw, gp);
     if (tiny) {
-      rows_edges<T, L, V, DROP>(a, ln, jj, ln.g * L, 0, 1, deg, wave_group_max<L>(deg), r.y, rh, st);
+      rows_edges<T, L, V, DROP, UM>(a, ln, jj, ln.g * L, 0, 1, deg, wave_group_max<L>(deg), r.y, rh, st);
     } else {
-      rows_edges<T, L, V, DROP>(a, ln, jj, 0, ln.g, G, deg, (deg + G - 1) / G, r.y, rh, st);
+      rows_edges<T, L, V, DROP, UM>(a, ln, jj, 0, ln.g, G, deg, (deg + G - 1) / G, r.y, rh, st);
       rows_group_sum<L, W, V>(st);
     }
     rows_dots<L, W, V>(ln, st, st.B, gp, cq, a.inv_h, wsum, A);
@@ -1030,7 +1037,7 @@ __global__ __launch_bounds__(kBlock) void gat_bwd_rows_fl_kernel(GatBwdArgs<T> a
     const int cnt = min(kWave, sg.z - tb);
     const int tn = tb + kSegRound + ln.lane;
     const int jn = tn < sg.z ? a.col[tn] : jj;
-    rows_edges<T, L, V, DROP>(a, ln, jj, 0, ln.g, G, cnt, (cnt + G - 1) / G, tb, rh, st);
+    rows_edges<T, L, V, DROP, UM>(a, ln, jj, 0, ln.g, G, cnt, (cnt + G - 1) / G, tb, rh, st);
     jj = jn;
   }
   rows_group_sum<L, W, V>(st);
@@ -2073,12 +2080,24 @@ int BwdFlLauncher<T, L, V>::run(hipStream_t st, const GatBwdArgs<T>& a, const Sc
       if (rc) return rc;
     }
   } else if (rb > 0) {
-    if (a.p > 0.0f)
-      hipLaunchKernelGGL((gat_bwd_rows_fl_kernel<T, L, V, true>), dim3(rb), dim3(kBlock), 0, st, a, rs, r_mid,
-                         r_mid_blocks, lgcq);
-    else
-      hipLaunchKernelGGL((gat_bwd_rows_fl_kernel<T, L, V, false>), dim3(rb), dim3(kBlock), 0, st, a, rs, r_mid,
-                         r_mid_blocks, lgcq);
+    auto launch = [&](auto UC) {
+      constexpr int UM = decltype(UC)::value;
+      if (a.p > 0.0f)
+        hipLaunchKernelGGL((gat_bwd_rows_fl_kernel<T, L, V, true, UM>), dim3(rb), dim3(kBlock), 0, st, a, rs, r_mid,
+                           r_mid_blocks, lgcq);
+      else
+        hipLaunchKernelGGL((gat_bwd_rows_fl_kernel<T, L, V, false, UM>), dim3(rb), dim3(kBlock), 0, st, a, rs, r_mid,
+                           r_mid_blocks, lgcq);
+    };
+    if constexpr (FlGeom<T>::W == 8 && V == 1) {
+      launch(std::integral_constant<int, kRowsUWide>());
+    } else if constexpr (FlGeom<T>::W == 8 && V < 8) {
+      // (the sums are in edge order for any batch: a shard has the bits of its graph)
+      if (a.n < kRowsUWideRows) launch(std::integral_constant<int, kRowsU>());
+      else launch(std::integral_constant<int, kRowsUWide>());
+    } else {
+      launch(std::integral_constant<int, kRowsU>());
+    }
     const int rc = check_launch("cign_gat_bwd (rows, feature layout)");
     if (rc) return rc;
   }
