@@ -163,8 +163,8 @@ class _CollapsedGATExt:
                  permute.data_ptr(), edge_max.data_ptr(), edge_sum.data_ptr(), edge_mask.data_ptr(),
                  in_feat.data_ptr(), attn_row.data_ptr(), attn_col.data_ptr(), pre.data_ptr(), grad_y.data_ptr(),
                  *rs.args(), rs.counters.data_ptr(), *cs.args(), cs.counters.data_ptr(), ws.data_ptr(), ws_bytes,
-                 *vectors, grad_feat.data_ptr(), grad_attn_row.data_ptr(), grad_attn_col.data_ptr(), grad_bias.data_ptr(),
-                 _lib.ptr(row_agg))
+                 *vectors, grad_feat.data_ptr(), grad_attn_row.data_ptr(), grad_attn_col.data_ptr(),
+                 grad_bias.data_ptr(), _lib.ptr(row_agg))
         return [grad_feat, grad_attn_row, grad_attn_col, grad_bias]
 
 

@@ -334,7 +334,7 @@ __device__ __forceinline__ void mfma_settle(f32x4 (&acc)[R][TN]) {
 }
 
 // One bf16 MFMA, or the four fp32 MFMAs of a 16-wide k chunk (k slices x, y,
-// z, w), accumulating into c: in place when ASM (operands from LDS reads).
+// z, w), accumulating into c: in place when ASM (operands as loads left them).
 template <bool ASM>
 __device__ __forceinline__ void mma_bf16(f32x4& c, const bf16x8& a, const bf16x8& b) {
   if constexpr (ASM) mfma_bf16_acc(c, a, b);
@@ -354,8 +354,10 @@ __device__ __forceinline__ void mma_f32x4(f32x4& c, const float4& a, const float
     c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, c, 0, 0, 0);
   }
 }
-// Kernels whose MFMA operands all come from LDS reads take the in-place
-// form whether or not their global loads are guarded.
+// Kernels whose MFMA operands are all registers that LDS or, for the W of
+// pack_proj_fwd16_kernel, global loads wrote take the in-place form whether or
+// not their global loads are guarded. An operand that a VALU instruction wrote
+// would need wait states of its own, which the compiler does not place for asm.
 constexpr bool kLdsAsm = CIGN_GEMM_ASM_MFMA;
 
 // MFMAs of one K step. The W tile is the MFMA's first operand and x the

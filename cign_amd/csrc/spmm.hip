@@ -101,16 +101,11 @@ namespace {
 #define CIGN_SPMM_WAVES 8
 #endif
 constexpr int kSpmmWaves = CIGN_SPMM_WAVES;
-// Chunks in flight per lane (a batch of U edges x VPL chunks), and the
-// smallest number of chunks a lane owns per row (more rows per wavefront).
+// Chunks in flight per lane (a batch of U edges x VPL chunks).
 #ifndef CIGN_SPMM_INFLIGHT
 #define CIGN_SPMM_INFLIGHT 8
 #endif
-#ifndef CIGN_SPMM_MIN_VPL
-#define CIGN_SPMM_MIN_VPL 1
-#endif
 constexpr int kSpmmInflight = CIGN_SPMM_INFLIGHT;
-constexpr int kSpmmMinVpl = CIGN_SPMM_MIN_VPL;
 constexpr int kSpmmBlock = kSpmmWaves * kWave;
 constexpr int kTile = 64;
 constexpr int kSegEdges = kSpmmWaves * kTile;
@@ -336,12 +331,12 @@ __global__ __launch_bounds__(kSpmmBlock) void spmm_kernel(SpmmArgs<T, W, VPL, TI
   }
 
   // Heavy-row segment: wave w takes the segment's edges [64w, 64w + 64) of
-  // every 256-edge round, reduced through LDS.
+  // every round of kSegEdges, reduced through LDS.
   __shared__ float red[kSpmmWaves][VPL * W * kWave];
   __shared__ int flag;
   const int4 sg = s.seg[b];
   const int row = sg.x;
-  // Rounds of 4 x 64 edges when the schedule's segments are longer than 256.
+  // Several rounds where the schedule's segments are longer than one.
   // The next round's indices and weights are loaded before this round's
   // gathers, so a round waits on one memory latency instead of two.
   int tb = sg.y + wave * kTile;
@@ -601,9 +596,11 @@ int cign_spmm(void* stream, int32_t dtype, int32_t n_rows, int32_t d, const int3
   if (n_rows < 0 || d <= 0) return set_error(kInvalid, "cign_spmm: bad sizes n_rows=%d d=%d", n_rows, d);
   if (!sched_info) return set_error(kInvalid, "cign_spmm: null schedule header");
   const SchedInfo info = read_info(sched_info);
-  if (info.n_light + info.n_hrow != n_rows) return set_error(kInvalid, "cign_spmm: schedule does not cover %d rows", n_rows);
+  if (info.n_light + info.n_hrow != n_rows)
+    return set_error(kInvalid, "cign_spmm: schedule does not cover %d rows", n_rows);
   if (!sched || !x || !y) return set_error(kInvalid, "cign_spmm: null pointer");
-  if (info.n_seg > 0 && (!partial || !counters)) return set_error(kInvalid, "cign_spmm: heavy rows need partial/counters");
+  if (info.n_seg > 0 && (!partial || !counters))
+    return set_error(kInvalid, "cign_spmm: heavy rows need partial/counters");
   const Sched s = make_sched(sched, info.n_light, info.n_seg, info.n_hrow);
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == kF32) return spmm_dispatch<float>(st, s, info, d, col, val, x, add, y, partial, counters);

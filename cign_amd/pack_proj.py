@@ -5,9 +5,10 @@ residual (generic_engine/model_cign.py:803-846 then :927-933):
     G   = cat_k alpha_k [W_k, D_k]           (never stored)
     out = h + gamma * dropout(G Wp^T + bp)
 
-cign_pack_proj_fwd builds G's tiles inside the projection's MFMA operands; cign_pack_proj_bwd computes grad_G tile by tile and runs the pack's
-backward on it in the same kernel, rebuilds G in the grad_Wp reduction, and
-adds the node gate's backward. Values and gradients are those of
+cign_pack_proj_fwd builds G's tiles inside the projection's MFMA operands;
+cign_pack_proj_bwd computes grad_G tile by tile and runs the pack's backward
+on it in the same kernel, rebuilds G in the grad_Wp reduction, and adds the
+node gate's backward. Values and gradients are those of
 gated_clifford_pack / clifford_pack_any followed by linear_gamma_residual,
 up to the order of the fp32 sums inside the products.
 """
