@@ -111,8 +111,8 @@ constexpr int kFwdUBig = CIGN_FL_FWD_U_BIG;
 // keep 16.
 constexpr int kFwdUNarrowF32 = 8;
 constexpr int kRowsU = CIGN_FL_ROWS_U;
-// Rows of 8-value (bf16) chunks: half of it, but the whole in rows of several
-// chunks a lane where there are few rows or they are the widest. The larger
+// Rows of 8-value (bf16) chunks: half of it, but the whole in rows of two or
+// three chunks a lane where there are few rows, and in rows of four. The larger
 // batch has fewer rounds and the registers of two wavefronts per SIMD; from
 // about 16K rows on the wavefronts the smaller one has room for are worth more.
 // GAT backward, us, 16 slots / 8: 6 x 256 at 2,000 nodes 52.5 / 55.1, 11,003
@@ -2091,7 +2091,7 @@ int BwdFlLauncher<T, L, V>::run(hipStream_t st, const GatBwdArgs<T>& a, const Sc
     };
     if constexpr (FlGeom<T>::W == 8 && V == 1) {
       launch(std::integral_constant<int, kRowsUWide>());
-    } else if constexpr (FlGeom<T>::W == 8 && V < 8) {
+    } else if constexpr (FlGeom<T>::W == 8 && V < 4) {
       // (the sums are in edge order for any batch: a shard has the bits of its graph)
       if (a.n < kRowsUWideRows) launch(std::integral_constant<int, kRowsU>());
       else launch(std::integral_constant<int, kRowsUWide>());

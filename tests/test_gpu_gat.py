@@ -494,3 +494,30 @@ def test_values_that_are_no_numbers_stay_with_their_neighbours(H, C, dtype, p, a
             (x2 if where == "features" else gy2)[0] = bad
             for k, v in results(x2, gy2).items():
                 assert torch.equal(v[1:], want[k][1:]), f"{k} with {bad} in node 0's {where}"
+
+
+@pytest.mark.parametrize("p", [0.0, 0.3])
+@pytest.mark.parametrize("H", [4, 6, 8])
+def test_wide_bf16_rows_gather_batches(H, p):
+    """The rows pass's batch of wide bf16 rows changes at 16,384 rows; sums are
+    in edge order for any batch, so one more node that is adjacent to itself
+    only leaves every bit of the others' results (two, three and four chunks a
+    lane)."""
+    from cign_amd.collapsed_gat import ensure_collapsed_gat_loaded
+
+    print(f"gat rows batches H={H} p={p}", flush=True)
+    rng = np.random.default_rng(H)
+    n, C = 16383, 256
+    ei = _graph(rng, n, {3: 1000, 7: 300})
+    x, ar, ac, b, gy = _inputs(rng, n + 1, H, C, torch.bfloat16)
+    ext = ensure_collapsed_gat_loaded()
+    runs = []
+    for m in (n, n + 1):
+        e = ei if m == n else np.concatenate([ei, [[n], [n]]], 1)
+        rowptr, col, row, colptr, perm = _dev_graph(e, m)
+        t = [v[:m] for v in (x, ar, ac, gy)]
+        out, pre, emax, esum, mask = ext.forward(t[1], t[2], rowptr, col, 0.2, t[0], b, p, 7)
+        runs.append(ext.backward(0.2, p, rowptr, col, colptr, row, perm, emax, esum, mask, t[0], t[1], t[2], pre, t[3],
+                                 None)[:3])
+    for name, a, c in zip(("grad_feat", "grad_attn_row", "grad_attn_col"), *runs):
+        assert torch.equal(a, c[:n]), name
