@@ -973,9 +973,16 @@ __device__ __forceinline__ void rows_emit(const GatBwdArgs<T>& a, const FlLane<L
   if (ln.qv[0] && ln.hq[0] == 0) store_f32<W>(a.grad_pre + static_cast<int64_t>(row) * a.gp_stride + ln.cw * W, gp);
 }
 
+// Wavefronts per SIMD that the compiler is held to: rows of three bf16 chunks a
+// lane with 16 slots had 165 VGPRs and three of them before padded shapes came
+// here, then 232 and two; held to three, 168 without spills (6 x 256, GAT
+// backward, us: 2,000 nodes 52.5 -> 50.4, 11,003 106.2 -> 103.6).
+template <typename T, int V, bool DROP, int UM>
+constexpr int kRowsWaves = std::is_same_v<T, bf16> && V == 3 && !DROP && UM == 16 ? 3 : 1;
+
 template <typename T, int L, int V, bool DROP, int UM>
-__global__ __launch_bounds__(kBlock) void gat_bwd_rows_fl_kernel(GatBwdArgs<T> a, Sched s, int n_mid, int mid_blocks,
-                                                                 int lgcq) {
+__global__ __launch_bounds__(kBlock, (kRowsWaves<T, V, DROP, UM>)) void gat_bwd_rows_fl_kernel(
+    GatBwdArgs<T> a, Sched s, int n_mid, int mid_blocks, int lgcq) {
   constexpr int W = FlGeom<T>::W;
   constexpr int G = kWave / L;
   const int cq = 1 << lgcq;
